@@ -13,18 +13,14 @@
 // (and rows of x).
 //
 // Device layout: the reference's row-major bytes, each row padded to a
-// multiple of 64 bytes.  A workgroup owns one 64-byte column tile of every row
-// (64 int8 columns, or 64 low- and 64 high-nibble int4 columns).  With several
-// rows of x (k_qlinear) it walks K in chunks of 512 rows: all 256 threads
-// stream a chunk (32 KB, row segments of 16 bytes) and its scaled activations
-// into one LDS buffer while wave i sums the previous chunk for x row i, one
-// lane per column, in ascending p.  With one row (k_qlinear_row, the decode
-// case) one wave sums and three form the products.  The sums are dependency
-// chains of K adds, so the columns (and rows of x) are the parallelism and the
-// chunk pipeline keeps the loads in flight meanwhile.
+// multiple of 64 bytes.  Several rows of x (a prompt) run on k_linear_seq
+// (fh_seq.hpp).  With one row (k_qlinear_row, the decode case) one wave sums
+// and three form the products.  The sums are dependency chains of K adds, so
+// the columns (and rows of x) are the parallelism and the chunk pipeline keeps
+// the loads in flight meanwhile.
 #include <type_traits>
 
-#include "fh_internal.hpp"
+#include "fh_seq.hpp"
 
 #pragma clang fp contract(off)
 
@@ -42,9 +38,7 @@ namespace {
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kTile = 64;    // column bytes per workgroup
-constexpr int kChunk = 512;  // rows p per LDS chunk
-constexpr int kSegs = kChunk * kTile / 16 / kThreads;  // 16-byte row segments per thread and chunk
+constexpr int kTile = 64;  // the rows' padding, in bytes
 
 // quant.rs:222-225 nibble_to_i8: sign-extend a 4-bit level
 __device__ __forceinline__ float level4(uint32_t b, bool hi) {
@@ -52,87 +46,56 @@ __device__ __forceinline__ float level4(uint32_t b, bool hi) {
     return static_cast<float>(static_cast<int8_t>(static_cast<uint8_t>(nib << 4)) >> 4);
 }
 
-// KIND 0: int8, 1: int4.  M rows of x per workgroup (grid.y over row groups),
-// one summing wave per row.
-template <int KIND, int M>
-__global__ void __launch_bounds__(kThreads)
-    k_qlinear(const uint8_t* __restrict__ q, const float* __restrict__ scales, const float* __restrict__ x,
-              const float* __restrict__ bias, float* __restrict__ y, int m, int k, int n, int pitch) {
-    static_assert(M <= kThreads / 64, "one summing wave per row");
-    __shared__ __align__(16) uint8_t wt[2][kChunk][kTile];
-    __shared__ float a[2][M][kChunk];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int c0 = blockIdx.x * kTile, row0 = blockIdx.y * M;
-    const int half = (n + 1) / 2;
-    // the column(s) lane `lane` of a summing wave owns
-    const int col_lo = c0 + lane, col_hi = half + c0 + lane;
-    const bool live_lo = KIND == 0 ? col_lo < n : col_lo < half;
-    const bool live_hi = KIND == 1 && col_hi < n;
-    const bool summing = wave < M && row0 + wave < m;
-    // every output starts at its bias (the reference fuses the bias first)
-    float acc_lo = bias && live_lo ? bias[col_lo] : 0.0f;
-    float acc_hi = bias && live_hi ? bias[col_hi] : 0.0f;
-    const int chunks = (k + kChunk - 1) / kChunk;
-    constexpr int kAPer = kChunk / kThreads;  // activation rows per thread and chunk
-    u4 seg[kSegs];
-    float xv[M][kAPer], sv[kAPer];
-    // Chunk c: thread t loads segment t % 4 of rows t / 4 + 64 j, and x and the
-    // scale of rows t + 256 j (all clamped to valid rows: rows past K are
-    // loaded, never summed).
-    auto fetch = [&](int c) __attribute__((always_inline)) {
-        const int p0 = c * kChunk;
-#pragma unroll
-        for (int j = 0; j < kSegs; j++) {
-            const int p = min(p0 + (tid >> 2) + j * (kThreads / 4), k - 1);
-            seg[j] = *reinterpret_cast<const u4*>(q + static_cast<size_t>(p) * pitch + c0 + (tid & 3) * 16);
-        }
-#pragma unroll
-        for (int j = 0; j < kAPer; j++) {
-            const int p = min(p0 + tid + j * kThreads, k - 1);
-            sv[j] = scales[p];
-#pragma unroll
-            for (int i = 0; i < M; i++) xv[i][j] = x[static_cast<size_t>(min(row0 + i, m - 1)) * k + p];
-        }
+// The levels for k_linear_seq: C output columns per workgroup are C bytes of
+// each int8 row, or C / 2 bytes of each int4 row (the first half of the columns
+// are the low nibbles', the second the high ones').  Thread t widens positions
+// 4 (t / 8) .. + 3 of the columns that piece t % 8 of those rows holds.
+template <int KIND, int COLS>
+struct LevelSrc {
+    static constexpr int C = COLS;
+    static constexpr bool kBiasFirst = true, kScaled = true;
+    static constexpr int kBytes = KIND == 0 ? C : C / 2;  // of a row per workgroup
+    static constexpr int kPiece = kBytes / 8;             // of a row per thread
+    using Piece = std::conditional_t<kPiece == 1, uint8_t, std::conditional_t<kPiece == 2, uint16_t, uint32_t>>;
+    const uint8_t* q;
+    const float* scales;
+    int pitch, half;
+    struct Raw {
+        Piece v[4];
     };
-    // a'[i, p] = x[i, p] * scale[p] (ops.rs:331-339) and the levels, into buffer b
-    auto store = [&](int b) __attribute__((always_inline)) {
+    __device__ __forceinline__ float scale(int p) const { return scales[p]; }
+    __device__ __forceinline__ int column(int tile, int c, int n) const {
+        if (KIND == 0) return tile * kBytes + c < n ? tile * kBytes + c : -1;
+        const int b = tile * kBytes + c % kBytes, j = c < kBytes ? b : half + b;
+        return b < half && j < n ? j : -1;
+    }
+    __device__ __forceinline__ void load(int tid, int tile, int c, int, int k, Raw& r) const {
+        const uint8_t* src = q + tile * kBytes + (tid & 7) * kPiece;
 #pragma unroll
-        for (int j = 0; j < kSegs; j++)
-            *reinterpret_cast<u4*>(&wt[b][(tid >> 2) + j * (kThreads / 4)][(tid & 3) * 16]) = seg[j];
+        for (int i = 0; i < 4; i++) {
+            const int p = min(c * fh_seq::kChunk + 4 * (tid >> 3) + i, k - 1);
+            r.v[i] = *reinterpret_cast<const Piece*>(src + static_cast<size_t>(p) * pitch);
+        }
+    }
+    __device__ __forceinline__ void store(int tid, int c, int k, const Raw& r, fh_seq::f4* wt) const {
+        const int g = tid >> 3, piece = tid & 7;
+        uint32_t v[4];
 #pragma unroll
-        for (int j = 0; j < kAPer; j++)
+        for (int i = 0; i < 4; i++) v[i] = c * fh_seq::kChunk + 4 * g + i < k ? r.v[i] : 0u;
 #pragma unroll
-            for (int i = 0; i < M; i++) a[b][i][tid + j * kThreads] = xv[i][j] * sv[j];
-    };
-    fetch(0);
-    store(0);
-    __syncthreads();
-    for (int c = 0; c < chunks; c++) {
-        const int b = c & 1;
-        if (c + 1 < chunks) fetch(c + 1);  // next chunk in flight during the sums
-        if (summing) {
-            const int pn = min(kChunk, k - c * kChunk);
-            const float* ar = a[b][wave];
-            for (int u = 0; u < pn; u++) {
-                const uint32_t wb = wt[b][u][lane];
-                const float ap = ar[u];
-                if (KIND == 0) {
-                    acc_lo = acc_lo + ap * static_cast<float>(static_cast<int8_t>(wb));
-                } else {
-                    acc_lo = acc_lo + ap * level4(wb, false);
-                    acc_hi = acc_hi + ap * level4(wb, true);
+        for (int h = 0; h < C / kBytes; h++)
+#pragma unroll
+            for (int e = 0; e < kPiece; e++) {
+                float l[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t byte = (v[i] >> (8 * e)) & 0xFFu;
+                    l[i] = KIND == 0 ? static_cast<float>(static_cast<int8_t>(byte)) : level4(byte, h == 1);
                 }
+                wt[g * C + h * kBytes + piece * kPiece + e] = fh_seq::f4{l[0], l[1], l[2], l[3]};
             }
-        }
-        if (c + 1 < chunks) store(b ^ 1);  // the other buffer: last read two chunks ago
-        __syncthreads();
     }
-    if (summing) {
-        float* yr = y + static_cast<size_t>(row0 + wave) * n;
-        if (live_lo) yr[col_lo] = acc_lo;
-        if (live_hi) yr[col_hi] = acc_hi;
-    }
-}
+};
 
 // One row of x (the decode case).  A sum is a chain of K dependent adds, so
 // the time of the kernel is K times the cost of one step of that chain.  Here
@@ -302,7 +265,7 @@ __global__ void __launch_bounds__(kThreads)
 template <int KIND>
 int launch(fh_ctx* ctx, const fh_qweight* w, const float* x, size_t m, const float* bias, float* y) {
     const unsigned gx = static_cast<unsigned>(w->pitch / kTile);
-    const int mi = static_cast<int>(m), ki = static_cast<int>(w->k), ni = static_cast<int>(w->n);
+    const int ki = static_cast<int>(w->k), ni = static_cast<int>(w->n);
     const int pi = static_cast<int>(w->pitch);
     if (m == 1) {
         // the narrowest tile that still keeps the grid within one workgroup per CU
@@ -316,8 +279,16 @@ int launch(fh_ctx* ctx, const fh_qweight* w, const float* x, size_t m, const flo
             hipLaunchKernelGGL((k_qlinear_row<KIND, 64>), dim3(gx), dim3(kThreads), 0, ctx->stream, w->q, w->scales,
                                x, bias, y, ki, ni, pi);
     } else {
-        hipLaunchKernelGGL((k_qlinear<KIND, 4>), dim3(gx, static_cast<unsigned>((m + 3) / 4)), dim3(kThreads), 0,
-                           ctx->stream, w->q, w->scales, x, bias, y, mi, ki, ni, pi);
+        auto go = [&](auto src) {
+            using Src = decltype(src);
+            fh_seq::launch(ctx, src, (w->row_bytes + Src::kBytes - 1) / Src::kBytes, x, m, bias, y, w->n, w->k);
+        };
+        // 32 columns per workgroup for vocabulary heads (longer pieces of each
+        // row: int4 50257 x 768 at m = 4 27.9 against 38.7 us), 16 for layers
+        // (more workgroups: 768 x 768 8.3 against 9.0)
+        const int half = static_cast<int>((w->n + 1) / 2);
+        if (w->n >= 32768) go(LevelSrc<KIND, 32>{w->q, w->scales, pi, half});
+        else go(LevelSrc<KIND, 16>{w->q, w->scales, pi, half});
     }
     FH_HIP(ctx, hipGetLastError());
     return FH_OK;

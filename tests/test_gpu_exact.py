@@ -105,3 +105,29 @@ def test_exact_and_fast_modes_agree_to_the_rounding_rule(fh, orc):
     w.free()
     mass = np.abs(x.astype(np.float64)) @ np.abs(orc.q8_0_to_ferrum_weight(raw, n, k).astype(np.float64))
     assert (np.abs(fast.astype(np.float64) - exact) <= 1e-5 * np.maximum(np.abs(exact), mass)).all()
+
+
+# One, two and four rows per lane (the launch rule takes more of them as the
+# tiles of 16 columns and 16 rows outnumber the CUs), each with a K that ends
+# inside a 128-position chunk or a 16-position piece of it, ragged rows and
+# columns.
+@pytest.mark.parametrize("m,n,k", [(16, 17, 128), (17, 16, 160), (33, 130, 352), (65, 4081, 96), (130, 4090, 160)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_exact_rows_per_lane_and_ragged_edges(fh, orc, m, n, k, f32):
+    import ferrum_hip
+
+    rng = np.random.default_rng(m + n + k)
+    k -= 7 if f32 else 0
+    x = rng.standard_normal((m, k), dtype=np.float32)
+    x[m // 2, k - 1], x[m - 1, 0], x[0] = np.inf, np.nan, -0.0
+    b = rng.standard_normal(n, dtype=np.float32)
+    if f32:
+        rows = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+        rows[n - 1, k - 1] = -np.inf
+        w, want = ferrum_hip.Q8_0Weight.upload_f32(fh, rows), orc.linear_forward(x, np.ascontiguousarray(rows.T), b)
+    else:
+        raw = orc.quantize_weight(n, k, m, 0.02)
+        w, want = ferrum_hip.Q8_0Weight.upload(fh, raw, n, k), reference(orc, x, raw, n, k, b)
+    got = ferrum_hip.linear_forward(fh, x, w, b, numerics=ferrum_hip.W8A32_EXACT)
+    w.free()
+    bits_equal(got, want)

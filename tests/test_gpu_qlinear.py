@@ -69,3 +69,35 @@ def test_qlinear_errors(fh, orc):
     with pytest.raises(ferrum_hip.FerrumHipError, match="unknown kind"):
         ferrum_hip.QWeight(fh, ow.scales, ow.q, 64, 10, 2)
     w.free()
+
+
+# One, two and four rows per lane and both tile widths of the kernel for
+# several rows, K ending inside a chunk and inside a 16-position piece, odd
+# widths (the int4 halves' last columns), a bias of -0 under products of -0 (no
+# padding may turn the sum to +0) and non-finite activations.
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("m,k,n", [(2, 15, 1), (16, 128, 33), (17, 129, 31), (40, 300, 2303), (66, 130, 4095),
+                                   (129, 97, 4097), (5, 70, 32769), (2, 33, 40001)])
+def test_qlinear_rows_per_lane_and_ragged_edges(fh, orc, kind, m, k, n):
+    import torch
+
+    import ferrum_hip
+
+    rng = np.random.default_rng(m * 7 + n + kind)
+    wf = (rng.standard_normal((k, n)) * 0.05).astype(np.float32)
+    wf[:, 0] = np.abs(wf[:, 0])
+    ow = orc.QWeight(wf, k, n, kind)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0], x[m - 1, k - 1] = -0.0, np.inf
+    b = (rng.standard_normal(n) * 0.1).astype(np.float32)
+    b[0] = -0.0
+    want = orc.qlinear(x, ow, b, threads=1)
+    assert np.signbit(want[0, 0]) and want[0, 0] == 0
+    w = ferrum_hip.QWeight(fh, ow.scales, ow.q, k, n, kind)
+    y = torch.full((m, n), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    ferrum_hip.qlinear_async(fh, w, dev(x), m, k, dev(b), n, y)
+    got = host(fh, y)
+    w.free()
+    nan = np.isnan(got) & np.isnan(want)
+    assert np.array_equal(np.where(nan, 0, got.view(np.uint32)), np.where(nan, 0, want.view(np.uint32)))
