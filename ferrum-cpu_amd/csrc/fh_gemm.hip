@@ -613,110 +613,127 @@ __global__ void __launch_bounds__(512)
 // One v_mfma_i32_32x32x32_i8 is one Q8_0 block of a 32 x 32 output tile: the
 // int32 block dots are exact; each is scaled and added to the f32 sum in
 // ascending b with separately rounded products and sums, the reference's own
-// order, so the outputs are the reference's bit for bit.  That per-block VALU
-// epilogue (convert, two products, add: 64 instructions per MFMA) bounds the
-// kernel, not the matrix cores.  Each wave owns a (32 TM) x 64 output tile and
-// reads its fragments straight from global memory: the activation panel
-// (fh_k_encode_panel) in MFMA lane order, 1 KiB contiguous per fragment; the
-// weight rows 16 bytes per lane.  The next block's operands are loaded while
-// the current one is finished.
-template <int TM, bool FAST>
-__global__ void __launch_bounds__(256)
-    k_gemm_w8a8(const uint4* __restrict__ qp, const float* __restrict__ dp, const int8_t* __restrict__ qs,
+// order, so the outputs are the reference's bit for bit.  The scale products
+// d_w * d_x of two blocks come from one v_mfma_f32_32x32x1_2b_f32 (its two
+// outer products are block b's and block b + 1's, 32 row scales by 32 column
+// scales; a product of two f16 values is exact in f32), which leaves three VALU
+// operations per output and block: convert, product, sum.  They bound the
+// kernel, not the matrix cores.
+// A workgroup owns a 64 x 64 tile, 2 x 2 waves of 32 x 32, and stages four Q8_0 blocks of K at a time through LDS (double buffered): the
+// activation panel (fh_k_encode_panel) is in MFMA lane order already, and a
+// weight row's four blocks are one 128-byte line read by eight lanes.  (With
+// every wave reading its own fragments from memory the L1's lookups bound the
+// kernel: a weight fragment is 32 pieces of 32 bytes.  3072 x 1024 at m = 511
+// ran 22.8 us so, 42.6 with a 64 x 64 tile per wave and 17.6 now.)  The 16-byte piece s of a
+// weight row r sits at slot r ^ s of its 32, so that the eight lanes that
+// store a row's pieces, and the eight that read one piece of eight rows, use
+// different banks.  Consecutive workgroups of an XCD take consecutive row
+// tiles of the same columns.
+constexpr int kW8Quad = 4;  // Q8_0 blocks per stage
+
+template <bool FAST>
+__global__ void __launch_bounds__(256, 2)
+    k_gemm_w8a8(const u4* __restrict__ qp, const float* __restrict__ dp, const int8_t* __restrict__ qs,
                 const uint16_t* __restrict__ dsc, const float* __restrict__ bias, float* __restrict__ y, int m, int n,
-                int k, int tiles_n, int tiles) {
+                int k, int tiles_m) {
     typedef int i4 __attribute__((ext_vector_type(4)));
     typedef int i16 __attribute__((ext_vector_type(16)));
-    constexpr int TN = 2;
-    const int lane = threadIdx.x & 63, g = lane >> 5, l32 = lane & 31;
-    const int wid = static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x >> 6);
-    if (wid >= tiles) return;  // no barriers below
-    const int tm = wid / tiles_n, tn = wid % tiles_n;
-    const int kb = k >> 5;
-    const int j0 = tn * 64;
-    const int8_t* wrow[TN];
-    const uint16_t* drow[TN];
+    typedef float f32x __attribute__((ext_vector_type(32)));
+    constexpr int NB = kW8Quad;  // blocks per stage
+    __shared__ __attribute__((aligned(16))) u4 s_a[2][2][NB][64], s_w[2][2][NB][64];
+    __shared__ float s_dx[2][2][NB][32], s_dw[2][2][NB][32];
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+    const int groups = static_cast<int>(gridDim.x), per_xcd = groups / 8, rem = groups % 8;
+    const int xcd = static_cast<int>(blockIdx.x) % 8, slot = static_cast<int>(blockIdx.x) / 8;
+    const int group = xcd * per_xcd + min(xcd, rem) + slot;
+    const int tm = group % tiles_m, j0 = group / tiles_m * 64;
+    const int kb = k >> 5, stages = (kb + NB - 1) / NB;
+
+    // Staging, per thread: two fragment pieces, piece tid % 8 of weight rows
+    // tid / 8 and tid / 8 + 32, a row scale and a weight scale (column tid / 4,
+    // block tid % 4).  Blocks past the last repeat it with zero scales; columns
+    // past n repeat column n - 1 (never stored).
+    const int wr = tid >> 3, ws = tid & 7;
+    const int8_t* wsrc[2];
 #pragma unroll
-    for (int c = 0; c < TN; c++) {
-        const int j = min(j0 + c * 32 + l32, n - 1);  // rows past n: computed, never stored
-        wrow[c] = qs + static_cast<size_t>(j) * k + g * 16;
-        drow[c] = dsc + static_cast<size_t>(j) * kb;
-    }
-    struct Ops {
-        i4 a[TM], w[TN];
-        f4 dx[TM][4];
-        uint16_t dw[TN];
+    for (int h = 0; h < 2; h++)
+        wsrc[h] = qs + static_cast<size_t>(min(j0 + 32 * h + wr, n - 1)) * k + (ws & 1) * 16;
+    const uint16_t* dsrc = dsc + static_cast<size_t>(min(j0 + (tid >> 2), n - 1)) * kb;
+    u4 ra[2], rw[2];
+    float rx;
+    uint16_t rd;
+    auto load = [&](int st) __attribute__((always_inline)) {
+        const int b0 = st * NB;
+#pragma unroll
+        for (int p = 0; p < 2; p++)
+            ra[p] = qp[(static_cast<size_t>(tm * 2 + p) * kb + min(b0 + wave, kb - 1)) * 64 + lane];
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+            rw[h] = *reinterpret_cast<const u4*>(wsrc[h] + min(b0 + (ws >> 1), kb - 1) * 32);
+        rx = dp[(static_cast<size_t>(tm * 2 + (tid >> 7)) * kb + min(b0 + ((tid >> 5) & 3), kb - 1)) * 32 + (tid & 31)];
+        rd = dsrc[min(b0 + (tid & 3), kb - 1)];
     };
-    auto load = [&](Ops& o, int b) __attribute__((always_inline)) {
+    auto store = [&](int st) __attribute__((always_inline)) {
+        const int buf = st & 1, b0 = st * NB;
 #pragma unroll
-        for (int r = 0; r < TM; r++) {
-            const size_t t = static_cast<size_t>(tm * TM + r) * kb + b;
-            o.a[r] = __builtin_bit_cast(i4, qp[t * 64 + lane]);
+        for (int p = 0; p < 2; p++) s_a[buf][p][wave][lane] = ra[p];
 #pragma unroll
-            for (int q = 0; q < 4; q++) o.dx[r][q] = *reinterpret_cast<const f4*>(dp + t * 32 + q * 8 + g * 4);
-        }
-#pragma unroll
-        for (int c = 0; c < TN; c++) {
-            o.w[c] = *reinterpret_cast<const i4*>(wrow[c] + b * 32);
-            o.dw[c] = drow[c][b];
-        }
+        for (int h = 0; h < 2; h++) s_w[buf][h][ws >> 1][(ws & 1) * 32 + (wr ^ ws)] = rw[h];
+        s_dx[buf][tid >> 7][(tid >> 5) & 3][tid & 31] = b0 + ((tid >> 5) & 3) < kb ? rx : 0.0f;
+        s_dw[buf][tid >> 7][tid & 3][(tid >> 2) & 31] = b0 + (tid & 3) < kb ? fh_h2f(rd) : 0.0f;
     };
-    float acc[TM][TN][16];
+    float acc[16];
 #pragma unroll
-    for (int r = 0; r < TM; r++)
-#pragma unroll
-        for (int c = 0; c < TN; c++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) acc[r][c][v] = 0.0f;
-    auto finish = [&](const Ops& o) __attribute__((always_inline)) {
+    for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+    auto finish = [&](int st) __attribute__((always_inline)) {
 #pragma clang fp contract(off)  // plain operators: separately rounded products and sums
+        const int buf = st & 1;
 #pragma unroll
-        for (int c = 0; c < TN; c++) {
-            const float dw = fh_h2f(o.dw[c]);
+        for (int h = 0; h < NB / 2; h++) {
+            const f32x dd = __builtin_amdgcn_mfma_f32_32x32x1f32(s_dx[buf][wm][2 * h + g][l32],
+                                                                 s_dw[buf][wn][2 * h + g][l32], f32x{}, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < TM; r++) {
-                const i16 d = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[r], o.w[c], i16{}, 0, 0, 0);
+            for (int i = 0; i < 2; i++) {
+                const int b = 2 * h + i;
+                const i4 w = __builtin_bit_cast(i4, s_w[buf][wn][b][g * 32 + (l32 ^ (2 * b + g))]);
+                const i4 a = __builtin_bit_cast(i4, s_a[buf][wm][b][lane]);
+                const i16 d = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w, i16{}, 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
-                    // acc row (v / 4) * 8 + g * 4 + v % 4: its scale is dx[v / 4][v % 4]
-                    const float dd = dw * o.dx[r][v >> 2][v & 3];
-                    if (FAST) acc[r][c][v] = __builtin_fmaf(static_cast<float>(d[v]), dd, acc[r][c][v]);
-                    else acc[r][c][v] = acc[r][c][v] + static_cast<float>(d[v]) * dd;
+                    const float t = static_cast<float>(d[v]);
+                    if (FAST) acc[v] = __builtin_fmaf(t, dd[16 * i + v], acc[v]);
+                    else acc[v] = acc[v] + t * dd[16 * i + v];
+                    asm volatile("" : "+v"(acc[v]));  // (keeps the sum before the fence below)
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);  // in order: bounds the live products
         }
     };
-    Ops o0, o1;
-    load(o0, 0);
-    for (int b = 0; b < kb; b += 2) {
-        if (b + 1 < kb) load(o1, b + 1);
-        finish(o0);
-        if (b + 1 >= kb) break;
-        if (b + 2 < kb) load(o0, b + 2);
-        finish(o1);
+    load(0);
+    store(0);
+    __syncthreads();
+    for (int st = 0; st < stages; st++) {
+        if (st + 1 < stages) load(st + 1);
+        finish(st);
+        if (st + 1 < stages) store(st + 1);  // (the other stage's readers finished before the last barrier)
+        __syncthreads();
     }
+    const int j = j0 + wn * 32 + l32;
+    if (j >= n) return;
+    const float bj = bias ? bias[j] : 0.0f;
 #pragma unroll
-    for (int c = 0; c < TN; c++) {
-        const int j = j0 + c * 32 + l32;
-        if (j >= n) continue;
-        const float bj = bias ? bias[j] : 0.0f;
-#pragma unroll
-        for (int r = 0; r < TM; r++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const int i = (tm * TM + r) * 32 + (v >> 2) * 8 + g * 4 + (v & 3);
-                if (i < m) y[static_cast<size_t>(i) * n + j] = bias ? acc[r][c][v] + bj : acc[r][c][v];
-            }
+    for (int v = 0; v < 16; v++) {
+        const int i = (tm * 2 + wm) * 32 + (v >> 2) * 8 + g * 4 + (v & 3);
+        if (i < m) y[static_cast<size_t>(i) * n + j] = bias ? acc[v] + bj : acc[v];
     }
 }
 
-// W8A8 for large m (a prompt's linears), the same arithmetic as k_gemm_w8a8
-// (every output the same bits), with the operands staged through LDS: a
-// workgroup owns a 256 x 256 output tile (eight waves of 128 x 64, 4 x 2
-// 32 x 32 tiles) and stages one Q8_0 block of it at a time.  Each operand byte
-// crosses from memory once per workgroup instead of once per wave.
-// The block terms are formed on the matrix cores, leaving two VALU
-// operations per output and block (the product and the sum):
+// W8A8 where 256 x 256 tiles fill the chip, the same arithmetic as k_gemm_w8a8
+// (every output the same bits): a workgroup owns a 256 x 256 output tile (eight
+// waves of 128 x 64, 4 x 2 32 x 32 tiles) and stages one Q8_0 block of it at a
+// time.  The block terms are formed on the matrix cores, leaving two VALU
+// operations per output and block, the product and the sum (FAST: one):
 //  * the int8 quants are staged as f16 (exact), and two
 //    v_mfma_f32_32x32x16_f16 give the block dot as an f32 that is the exact
 //    integer (|dot| <= 32 * 128 * 128 < 2^24, so every partial sum is
@@ -741,7 +758,6 @@ constexpr int kW8Rows = 256, kW8Cols = 256, kW8Threads = 512;
 constexpr int kW8BPlane = 260;  // 16-byte entries (padded: see the block-scaled kernel)
 constexpr int kW8BOff = 16 * 1024, kW8SOff = kW8BOff + 4 * kW8BPlane * 16;
 constexpr int kW8StageBytes = kW8SOff + 256 * 4 + 256 * 4;
-constexpr size_t kW8LdsMinRows = 1024;  // m from which W8A8 takes the staged kernel
 
 template <bool FAST>
 __global__ void __launch_bounds__(kW8Threads)
@@ -1702,12 +1718,20 @@ __global__ void fh_k_encode_panel(const float* __restrict__ x, int m, int m_pad,
                                   float* __restrict__ dp);
 
 // W8A8 through the int8 matrix cores: the activations are encoded into the
-// lane-order panel, then one wave per (32 TM) x 64 output tile.
+// lane-order panel, then the GEMM.
 int fh_launch_gemm_w8a8(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const float* bias, float* y,
                         bool fast) {
-    // (a prompt's m takes the LDS-staged kernel: its panel covers whole 256-row tiles)
-    const bool staged = m >= kW8LdsMinRows;
-    const int tm_rows = staged ? kW8Rows : m >= 64 ? 64 : 32;
+    // Two kernels, the one with the least time.  Measured (ns per block of K, 256
+    // CUs): the 64 x 64 workgroup tile 250 + 0.13 per 32 x 32 of output; the 256 x
+    // 256 one 2300 per round of one workgroup per CU, 2100 in the fast mode.  4096
+    // x 1024 at m = 4096 (one round): 80.4 us and 82.1, fast 77.0 and 69.2; 1024 x
+    // 4096 at m = 16352 (one round): 322.9 and 307.2; 768 x 3072 at m = 2048 (24
+    // tiles of 256 x 256 for the 256 CUs): 39.9 and 190.
+    const size_t cus = static_cast<size_t>(ctx->num_cus);
+    const size_t t32 = (m + 31) / 32 * ((w->n + 31) / 32);
+    const size_t t256 = (m + kW8Rows - 1) / kW8Rows * ((w->n + kW8Cols - 1) / kW8Cols);
+    const bool staged = (t256 + cus - 1) / cus * (fast ? 2100 : 2300) < 250 + t32 * 130 / 1000;
+    const int tm_rows = staged ? kW8Rows : 64;
     const size_t kb = w->k / 32, m_pad = (m + tm_rows - 1) / tm_rows * tm_rows;
     const size_t qbytes = fh_align256(m_pad * w->k), dbytes = fh_align256(m_pad * kb * 4);
     void* ws = nullptr;
@@ -1727,27 +1751,20 @@ int fh_launch_gemm_w8a8(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m,
     if (staged) {
         const size_t tn = (w->n + kW8Cols - 1) / kW8Cols, tl = tn * (m_pad / kW8Rows);
         if (tl > 0x7FFFFFFFu) return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: output above 2^31 tiles");
-        if (fast)
-            hipLaunchKernelGGL(k_gemm_w8a8_lds<true>, dim3(static_cast<unsigned>(tl)), dim3(kW8Threads), 0,
-                               ctx->stream, qp, dp, w->qs, w->d, bias, y, static_cast<int>(m),
-                               static_cast<int>(w->n), static_cast<int>(w->k), static_cast<int>(tn));
-        else
-            hipLaunchKernelGGL(k_gemm_w8a8_lds<false>, dim3(static_cast<unsigned>(tl)), dim3(kW8Threads), 0,
-                               ctx->stream, qp, dp, w->qs, w->d, bias, y, static_cast<int>(m),
-                               static_cast<int>(w->n), static_cast<int>(w->k), static_cast<int>(tn));
+        hipLaunchKernelGGL((fast ? k_gemm_w8a8_lds<true> : k_gemm_w8a8_lds<false>), dim3(static_cast<unsigned>(tl)),
+                           dim3(kW8Threads), 0, ctx->stream, qp, dp, w->qs, w->d, bias, y, static_cast<int>(m),
+                           static_cast<int>(w->n), static_cast<int>(w->k), static_cast<int>(tn));
         FH_HIP(ctx, hipGetLastError());
         return FH_OK;
     }
-    const size_t tiles_n = (w->n + 63) / 64, tiles = tiles_n * (m_pad / tm_rows);
-    if (tiles > 0x7FFFFFFFu) return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: output above 2^31 tiles");
-    const dim3 grid(static_cast<unsigned>((tiles + 3) / 4)), block(256);
+    const size_t tiles_m = m_pad / tm_rows, groups = (w->n + 63) / 64 * tiles_m;
+    if (groups > 0x7FFFFFFFu) return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: output above 2^31 tiles");
     auto go = [&](auto kern) {
-        hipLaunchKernelGGL(kern, grid, block, 0, ctx->stream, qp, dp, w->qs, w->d, bias, y, static_cast<int>(m),
-                           static_cast<int>(w->n), static_cast<int>(w->k), static_cast<int>(tiles_n),
-                           static_cast<int>(tiles));
+        hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(groups)), dim3(256), 0, ctx->stream,
+                           reinterpret_cast<const u4*>(qp), dp, w->qs, w->d, bias, y, static_cast<int>(m), static_cast<int>(w->n), static_cast<int>(w->k),
+                           static_cast<int>(tiles_m));
     };
-    if (tm_rows == 64) fast ? go(k_gemm_w8a8<2, true>) : go(k_gemm_w8a8<2, false>);
-    else fast ? go(k_gemm_w8a8<1, true>) : go(k_gemm_w8a8<1, false>);
+    fast ? go(k_gemm_w8a8<true>) : go(k_gemm_w8a8<false>);
     FH_HIP(ctx, hipGetLastError());
     return FH_OK;
 }

@@ -38,10 +38,12 @@ namespace {
 
 constexpr int kWaves = 4;  // waves per block of the GEMV with the LayerNorm prologue (the plain GEMV: one)
 constexpr int kLnMaxK = 2048;  // widest row the GEMV's LayerNorm prologue takes
-// W8A8 runs on the int8 matrix cores (one wave per 32- or 64-row x 64-column
-// output tile, every Q8_0 block in order) once there are this many tiles;
-// fewer waves, each walking all of K, lose to the block-parallel kernel below.
-constexpr size_t kW8a8MfmaTiles = 96;
+// W8A8 runs on the int8 matrix cores (every Q8_0 block of an output in order)
+// from this many outputs, or this many tiles of (32 or 64) x 64; fewer waves,
+// each walking all of K, lose to the block-parallel kernel below (768 x 3072:
+// 19.3 against 26.4 us at m = 64, 32.6 against 26.8 at 128; 2304 x 768: 10.4
+// against 10.9 at 32, 15.4 against 11.7 at 64).
+constexpr size_t kW8a8MfmaOutputs = 96 * 1024, kW8a8MfmaTiles = 96;
 
 __device__ __forceinline__ float sbyte(uint32_t w, int i) {
     return static_cast<float>(static_cast<int8_t>((w >> (8 * i)) & 0xFFu));
@@ -458,7 +460,8 @@ int fh_launch_linear_w8a8(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t 
     if (w->n > 0x7FFFFFFFu || w->k > 0x7FFFFFFFu || m * w->n > 0x7FFFFFFFu * size_t(64))
         return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: problem too large for the W8A8 kernel");
     const size_t tile_rows = m >= 64 ? 64 : 32;
-    if (m >= 32 && (m + tile_rows - 1) / tile_rows * ((w->n + 63) / 64) >= kW8a8MfmaTiles)
+    if ((m >= 8 && m * w->n >= kW8a8MfmaOutputs) ||
+        (m >= 32 && (m + tile_rows - 1) / tile_rows * ((w->n + 63) / 64) >= kW8a8MfmaTiles))
         return fh_launch_gemm_w8a8(ctx, w, x, m, bias, y, fast);
     const size_t kb = w->k / 32;
     const size_t qbytes = fh_align256(m * w->k), dbytes = fh_align256(m * kb * 2);

@@ -679,3 +679,27 @@ def test_q8_0_dequant_is_bit_exact(fh, orc):
     ferrum_hip.q8_0_dequant_async(fh, dr, 32 * 5000, out)
     fh.sync()
     assert np.array_equal(out.cpu().numpy().view(np.uint32), orc.q8_0_dequant(raw, 32 * 5000).view(np.uint32))
+
+
+# The int8 matrix-core kernels' edges: one and odd block counts (K is walked in
+# pairs, four pairs in flight), ragged rows and columns, one and two 32-row
+# tiles per wave and the LDS-staged kernel, non-finite scales on either side:
+# the reference's bits.
+@pytest.mark.parametrize("m,n,k", [(8, 12321, 32), (33, 3010, 96), (127, 801, 288), (511, 1024, 160), (6081, 1, 64),
+                                   (1000, 3073, 96), (2050, 2000, 224), (1025, 16129, 64)])
+def test_w8a8_pairs_of_blocks_are_bit_exact(fh, orc, m, n, k):
+    import ferrum_hip
+
+    raw = orc.quantize_weight(n, k, m + n, 0.05)
+    blocks = raw.reshape(n, k // 32, 34)
+    blocks[n // 2, -1, :2] = np.array([np.inf], np.float16).view(np.uint8)
+    x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
+    x[m // 2, k - 1], x[m - 1, 0] = np.inf, np.nan
+    b = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    w = ferrum_hip.Q8_0Weight.upload(fh, raw, n, k)
+    got = ferrum_hip.linear_forward(fh, x, w, b, numerics=ferrum_hip.W8A8)
+    w.free()
+    rows = sorted({0, 1, m // 3, m // 2, m - 2, m - 1} | set(range(m))) if m * n * k < 3e8 else \
+        [0, 31, 32, 63, 64, m // 2, 255 % m, 256 % m, m - 2, m - 1]
+    ref = orc.q8_0_linear_w8a8(x[rows], raw, n, b)
+    assert np.array_equal(got[rows], ref, equal_nan=True)
