@@ -196,6 +196,15 @@ int fh_ctx_create(int device, fh_ctx** out) {
         return code;
     }
     c->status = static_cast<unsigned*>(st);
+    // The split GEMMs' arrival counters (at most one per two CUs): there from the
+    // start, so that no GEMM has to grow them under graph capture.
+    void* counters = nullptr;
+    const int rc = fh_counter_area(c, static_cast<size_t>(c->num_cus) * 2, &counters);
+    if (rc) {
+        const std::string why = c->err;
+        fh_ctx_destroy(c);
+        return fh_fail(nullptr, rc, "fh_ctx_create (counters): " + why);
+    }
     *out = c;
     return FH_OK;
 }

@@ -26,11 +26,11 @@
 // read); the large-m block-scaled kernel (k_gemm_bscale) instead takes only
 // the row scales (k_row_scales, one read of x) and splits the activations
 // while staging them, which saves the panel's write and re-read.  k_gemm_mfma stages
-// KW Q8_0 blocks of the activation panel and of the weight rows per step into
+// a Q8_0 block of the activation panel and of the weight rows per step into
 // LDS (double buffered, one barrier per step), converting the int8 quants to
-// f16 on the way in; each wave owns TM x TN 32x32 output tiles, and with
-// KW > 1 the waves split the K blocks and add their sums in wave order (a
-// fixed order: results do not depend on timing).
+// f16 on the way in; each wave owns TM x TN 32x32 output tiles.  Up to some
+// thousands of 32 x 32 output tiles the skinny kernel takes the call in tiles
+// of rows (fh_launch_gemm_w8a32).
 #include "fh_internal.hpp"
 
 namespace {
@@ -236,78 +236,71 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Workgroup tile BM x BN; NW = WM x WN x KW waves (output sub-tiles x
-// K-slices).  Tiles are numbered so that consecutive workgroups on one XCD
+// Workgroup tile BM x BN, WM x WN waves, one block of K per step.  (At least two
+// waves per SIMD in the launch bounds: with room for one, the compiler gives the
+// matrix results accumulator registers that the vector units cannot read, a move
+// per value; 2304 x 768 at m = 1024, in 64 x 64 tiles, ran 46.8 us so and 28.5
+// without.)  Tiles are numbered so that consecutive workgroups on one XCD
 // (the hardware deals workgroup ids round-robin over the 8 XCDs) take
 // consecutive tiles of one activation row-tile, which then stays in that XCD's L2.
-template <int BM, int BN, int WM, int WN, int KW>
-__global__ void __launch_bounds__(64 * WM * WN * KW)
+template <int BM, int BN, int WM, int WN>
+__global__ void __launch_bounds__(64 * WM * WN, 2)
     k_gemm_mfma(const uint4* __restrict__ panel, const float* __restrict__ xinv, const float* __restrict__ x,
                 const int8_t* __restrict__ qs, const uint16_t* __restrict__ dsc, const int8_t* __restrict__ rexp,
-                const float* __restrict__ bias, float* __restrict__ y, int m, int n, int k, int tiles_n) {
-    constexpr int NW = WM * WN * KW, NT = 64 * NW;
+                const float* __restrict__ bias, float* __restrict__ y, int m, int n, int k, int tiles_n, int act) {
+    constexpr int NW = WM * WN, NT = 64 * NW;
     static_assert(NW == 4 || NW == 8, "four or eight waves");
     constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN);
     static_assert(TM >= 1 && TN >= 1 && TM * 32 * WM == BM && TN * 32 * WN == BN, "tile shape");
-    constexpr int A_BYTES = KW * BM * kArow * 2, B_BYTES = KW * BN * kBrow * 2, S_BYTES = KW * BN * 4;
+    constexpr int A_BYTES = BM * kArow * 2, B_BYTES = BN * kBrow * 2, S_BYTES = BN * 4;
     constexpr int STAGE = A_BYTES + B_BYTES + S_BYTES;
     // 16-byte pieces per thread (the last weight round may leave threads idle)
-    constexpr int AP = KW * BM * 8 / NT, BPN = KW * BN * 2, BP = (BPN + NT - 1) / NT;
-    static_assert(AP * NT == KW * BM * 8 && KW * BN <= NT, "staging split");
-    constexpr int RED = (KW - 1) * WM * WN * TM * TN * 16 * 64 * 4;
-    static_assert(RED + BM * 4 <= 2 * STAGE, "reduction and row scales fit the stage buffers");
+    constexpr int AP = BM * 8 / NT, BPN = BN * 2, BP = (BPN + NT - 1) / NT;
+    static_assert(AP * NT == BM * 8 && BN <= NT && BM * 4 <= 2 * STAGE, "staging split, row scales");
     __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int kw = wave / (WM * WN), wm = (wave % (WM * WN)) / WN, wn = wave % WN;
+    const int wm = wave / WN, wn = wave % WN;
     const int tiles = static_cast<int>(gridDim.x), per_xcd = tiles / 8, rem = tiles % 8;
     const int xcd = static_cast<int>(blockIdx.x) % 8, slot = static_cast<int>(blockIdx.x) / 8;
     const int tile = xcd * per_xcd + min(xcd, rem) + slot;  // XCDs 0 .. rem-1 take one extra tile
     const int tile_m = tile / tiles_n, tile_n = tile % tiles_n;
     const int j0 = tile_n * BN;
-    const int kb = k >> 5, steps = (kb + KW - 1) / KW;
-    const uint4* pan = panel + static_cast<size_t>(tile_m) * kb * BM * 8;
+    const int kb = k >> 5;
+    const u4* pan = reinterpret_cast<const u4*>(panel) + static_cast<size_t>(tile_m) * kb * BM * 8;
 
-    uint4 ra[AP], rb[BP];
+    u4 ra[AP], rb[BP];
     float rs = 0.0f;
-    auto load = [&](int st) __attribute__((always_inline)) {
+    auto load = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
-        for (int p = 0; p < AP; p++) {
-            const int piece = tid + NT * p, blk = piece / (BM * 8), rem = piece % (BM * 8);
-            const int b = st * KW + blk;
-            ra[p] = b < kb ? pan[static_cast<size_t>(b) * BM * 8 + rem] : make_uint4(0, 0, 0, 0);
-        }
+        for (int p = 0; p < AP; p++) ra[p] = pan[static_cast<size_t>(b) * BM * 8 + tid + NT * p];
 #pragma unroll
         for (int p = 0; p < BP; p++) {
-            const int piece = tid + NT * p, blk = piece / (BN * 2), rem = piece % (BN * 2);
-            const int b = st * KW + blk, j = j0 + rem / 2;
-            rb[p] = (piece < BPN && b < kb && j < n)
-                        ? *reinterpret_cast<const uint4*>(qs + static_cast<size_t>(j) * k + b * 32 + (rem & 1) * 16)
-                        : make_uint4(0, 0, 0, 0);
+            const int piece = tid + NT * p, j = j0 + piece / 2;
+            rb[p] = (piece < BPN && j < n)
+                        ? *reinterpret_cast<const u4*>(qs + static_cast<size_t>(j) * k + b * 32 + (piece & 1) * 16)
+                        : u4{0, 0, 0, 0};
         }
-        if (tid < KW * BN) {
-            const int b = st * KW + tid / BN, j = j0 + tid % BN;
-            rs = (b < kb && j < n) ? fh_h2f(dsc[static_cast<size_t>(j) * kb + b]) : 0.0f;
-        }
+        if (tid < BN) rs = j0 + tid < n ? fh_h2f(dsc[static_cast<size_t>(j0 + tid) * kb + b]) : 0.0f;
     };
     auto store = [&](int buf) __attribute__((always_inline)) {
         char* st = lds + buf * STAGE;
 #pragma unroll
         for (int p = 0; p < AP; p++) {
-            const int piece = tid + NT * p, blk = piece / (BM * 8), rem = piece % (BM * 8);
-            *reinterpret_cast<uint4*>(st + ((blk * BM + rem / 8) * kArow) * 2 + (rem % 8) * 16) = ra[p];
+            const int piece = tid + NT * p;
+            *reinterpret_cast<u4*>(st + (piece / 8 * kArow) * 2 + (piece % 8) * 16) = ra[p];
         }
 #pragma unroll
         for (int p = 0; p < BP; p++) {
-            const int piece = tid + NT * p, blk = piece / (BN * 2), rem = piece % (BN * 2);
+            const int piece = tid + NT * p;
             if (BPN % NT != 0 && piece >= BPN) break;
-            char* dst = st + A_BYTES + ((blk * BN + rem / 2) * kBrow) * 2 + (rem & 1) * 32;
+            char* dst = st + A_BYTES + (piece / 2 * kBrow) * 2 + (piece & 1) * 32;
             const uint2 a = quants_to_f16(rb[p].x), b = quants_to_f16(rb[p].y);
             const uint2 c = quants_to_f16(rb[p].z), d = quants_to_f16(rb[p].w);
             *reinterpret_cast<uint4*>(dst) = make_uint4(a.x, a.y, b.x, b.y);
             *reinterpret_cast<uint4*>(dst + 16) = make_uint4(c.x, c.y, d.x, d.y);
         }
-        if (tid < KW * BN) reinterpret_cast<float*>(st + A_BYTES + B_BYTES)[tid] = rs;
+        if (tid < BN) reinterpret_cast<float*>(st + A_BYTES + B_BYTES)[tid] = rs;
     };
 
     f16x acc[TM][TN];
@@ -321,13 +314,13 @@ __global__ void __launch_bounds__(64 * WM * WN * KW)
     store(0);
     __syncthreads();
     const int arow = lane % 32, koff = (lane / 32) * 8;
-    for (int st = 0; st < steps; st++) {
-        const int buf = st & 1;
-        if (st + 1 < steps) load(st + 1);
+    for (int b = 0; b < kb; b++) {
+        const int buf = b & 1;
+        if (b + 1 < kb) load(b + 1);
         const char* sb = lds + buf * STAGE;
-        const _Float16* As = reinterpret_cast<const _Float16*>(sb) + kw * BM * kArow;
-        const _Float16* Bs = reinterpret_cast<const _Float16*>(sb + A_BYTES) + kw * BN * kBrow;
-        const float* Ss = reinterpret_cast<const float*>(sb + A_BYTES + B_BYTES) + kw * BN;
+        const _Float16* As = reinterpret_cast<const _Float16*>(sb);
+        const _Float16* Bs = reinterpret_cast<const _Float16*>(sb + A_BYTES);
+        const float* Ss = reinterpret_cast<const float*>(sb + A_BYTES + B_BYTES);
         // Weight fragments and scales for all column tiles, then one row tile
         // at a time (its four activation fragments, then its MFMAs).
         h8 bq[TN][2];
@@ -335,9 +328,9 @@ __global__ void __launch_bounds__(64 * WM * WN * KW)
 #pragma unroll
         for (int c = 0; c < TN; c++) {
             const int col = (wn * TN + c) * 32 + arow;
-            const _Float16* b = Bs + col * kBrow + koff;
-            bq[c][0] = *reinterpret_cast<const h8*>(b);
-            bq[c][1] = *reinterpret_cast<const h8*>(b + 16);
+            const _Float16* bc = Bs + col * kBrow + koff;
+            bq[c][0] = *reinterpret_cast<const h8*>(bc);
+            bq[c][1] = *reinterpret_cast<const h8*>(bc + 16);
             dw[c] = Ss[col];
         }
 #pragma unroll
@@ -355,66 +348,37 @@ __global__ void __launch_bounds__(64 * WM * WN * KW)
                 for (int v = 0; v < 16; v++) acc[r][c][v] = fmaf(dw[c], p[v], acc[r][c][v]);
             }
         }
-        if (st + 1 < steps) store(buf ^ 1);
+        if (b + 1 < kb) store(buf ^ 1);
         __syncthreads();
-    }
-
-    if (KW > 1) {
-        // K-slices 1..KW-1 hand their sums to slice 0 through LDS; slice 0 adds
-        // them in slice order.
-        float* red = reinterpret_cast<float*>(lds);
-        const int sub = wave % (WM * WN);
-        if (kw > 0) {
-#pragma unroll
-            for (int r = 0; r < TM; r++)
-#pragma unroll
-                for (int c = 0; c < TN; c++)
-#pragma unroll
-                    for (int v = 0; v < 16; v++)
-                        red[((((kw - 1) * WM * WN + sub) * TM + r) * TN + c) * 1024 + v * 64 + lane] = acc[r][c][v];
-        }
-        __syncthreads();
-        if (kw == 0) {
-#pragma unroll
-            for (int s = 1; s < KW; s++)
-#pragma unroll
-                for (int r = 0; r < TM; r++)
-#pragma unroll
-                    for (int c = 0; c < TN; c++)
-#pragma unroll
-                        for (int v = 0; v < 16; v++)
-                            acc[r][c][v] += red[((((s - 1) * WM * WN + sub) * TM + r) * TN + c) * 1024 + v * 64 + lane];
-        }
     }
 
     // Row scales of this tile through LDS (the stage buffers are free).
     const int i0 = tile_m * BM;
-    float* s_inv = reinterpret_cast<float*>(lds) + RED / 4;
+    float* s_inv = reinterpret_cast<float*>(lds);
     __syncthreads();
     for (int t = tid; t < BM; t += NT) s_inv[t] = xinv[i0 + t];  // rows < m_pad
     __syncthreads();
-    if (KW == 1 || kw == 0) {  // K-slice 0 holds the totals
 #pragma unroll
-        for (int c = 0; c < TN; c++) {
-            const int j = j0 + (wn * TN + c) * 32 + arow;
-            if (j >= n) continue;
-            const float bj = bias ? bias[j] : 0.0f;
+    for (int c = 0; c < TN; c++) {
+        const int j = j0 + (wn * TN + c) * 32 + arow;
+        if (j >= n) continue;
+        const float bj = bias ? bias[j] : 0.0f;
 #pragma unroll
-            for (int r = 0; r < TM; r++)
+        for (int r = 0; r < TM; r++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int il = (wm * TM + r) * 32 + (v / 4) * 8 + (lane / 32) * 4 + (v % 4), i = i0 + il;
-                    if (i >= m) continue;
-                    const float s = acc[r][c][v] * s_inv[il];
-                    y[static_cast<size_t>(i) * n + j] = bias ? s + bj : s;
-                }
-        }
+            for (int v = 0; v < 16; v++) {
+                const int il = (wm * TM + r) * 32 + (v / 4) * 8 + (lane / 32) * 4 + (v % 4), i = i0 + il;
+                if (i >= m) continue;
+                const float s = acc[r][c][v] * s_inv[il];
+                const float o = bias ? s + bj : s;
+                y[static_cast<size_t>(i) * n + j] = act == FH_ACT_GELU ? gelu_unfused(o) : o;
+            }
     }
     // Rare: weight rows with a non-finite scale are rewritten with the
     // reference's own arithmetic (inf/NaN activations propagate exactly here).
     bool flagged = false;
     for (int t = tid; t < BN; t += NT) flagged |= j0 + t < n && rexp[j0 + t] == kFhBadRowExp;
-    if (__syncthreads_or(flagged)) exact_tile(x, qs, dsc, rexp, nullptr, bias, y, m, n, k, i0, j0, BM, BN, FH_ACT_NONE);
+    if (__syncthreads_or(flagged)) exact_tile(x, qs, dsc, rexp, nullptr, bias, y, m, n, k, i0, j0, BM, BN, act);
 }
 
 // ---- large m, block-scaled: the quants as the weight operand -------------------------
@@ -977,6 +941,14 @@ __global__ void __launch_bounds__(512)
     k_gemm_skinny(const float* __restrict__ x, const int8_t* __restrict__ qs, const uint16_t* __restrict__ dsc,
                   const int8_t* __restrict__ rexp, const float* __restrict__ bias, float* y, int m, int n,
                   int k, int bps, float* __restrict__ part, unsigned* __restrict__ counters, int act, fh_edge e) {
+    if constexpr (MODE == kSkinnyPlain) {  // grid.z: tiles of 32 MT rows (one in the other modes)
+        const size_t rows = static_cast<size_t>(blockIdx.z) * (32 * MT);
+        x += rows * k;
+        y += rows * n;
+        m -= static_cast<int>(rows);
+        part += static_cast<size_t>(blockIdx.z) * gridDim.y * gridDim.x * (MT * NT * 1024);
+        counters += static_cast<size_t>(blockIdx.z) * gridDim.x;
+    }
     constexpr int OUT = MT * NT * 1024;  // outputs of one workgroup
     // Per wave, [SLOT] floats: during the K loop one Q8_0 block of its
     // activation rows ([MT * 32][36]: the rows land there from row-contiguous
@@ -1531,8 +1503,8 @@ int launch_bscale(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const
     return FH_OK;
 }
 
-template <int BM, int BN, int WM, int WN, int KW>
-int launch_gemm(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const float* bias, float* y) {
+template <int BM, int BN, int WM, int WN>
+int launch_gemm(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const float* bias, float* y, int act) {
     const size_t m_pad = (m + BM - 1) / BM * BM;
     const size_t pbytes = fh_align256(m_pad * w->k * 4), ibytes = fh_align256(m_pad * 4), fbytes = fh_align256(m_pad);
     void* ws = nullptr;
@@ -1546,10 +1518,10 @@ int launch_gemm(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const f
     FH_HIP(ctx, hipGetLastError());
     const size_t tiles_n = (w->n + BN - 1) / BN, tiles = tiles_n * (m_pad / BM);
     if (tiles > 0x7FFFFFFFu) return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: output above 2^31 tiles");
-    hipLaunchKernelGGL((k_gemm_mfma<BM, BN, WM, WN, KW>), dim3(static_cast<unsigned>(tiles)),
-                           dim3(64 * WM * WN * KW), 0, ctx->stream, panel, xinv, x, w->qs, w->d, w->rexp, bias, y,
+    hipLaunchKernelGGL((k_gemm_mfma<BM, BN, WM, WN>), dim3(static_cast<unsigned>(tiles)),
+                           dim3(64 * WM * WN), 0, ctx->stream, panel, xinv, x, w->qs, w->d, w->rexp, bias, y,
                            static_cast<int>(m), static_cast<int>(w->n), static_cast<int>(w->k),
-                           static_cast<int>(tiles_n));
+                           static_cast<int>(tiles_n), act);
     FH_HIP(ctx, hipGetLastError());
     return FH_OK;
 }
@@ -1567,17 +1539,20 @@ __global__ void k_zero_counters(unsigned* __restrict__ c, int n) {
 
 template <int MT, int NT, int BPW>
 int launch_skinny_t(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const float* bias, float* y,
-                    const fh_scratch* scratch, int act, const fh_edge* edge = nullptr, int mode = kSkinnyPlain) {
+                    const fh_scratch* scratch, int act, const fh_edge* edge = nullptr, int mode = kSkinnyPlain,
+                    size_t max_waves = 0) {
     const size_t kb = w->k / 32, tiles = (w->n + 32 * NT - 1) / (32 * NT);
+    const size_t rows = (m + 32 * MT - 1) / (32 * MT);  // row tiles (one for m <= 32 MT)
     // Waves per workgroup: eight, except that a tile of more than two 32 x 32
     // output groups keeps 16 KB of wave sums per wave in LDS, so where the
     // tiles outnumber the CUs it takes four and two workgroups share a CU.
     // (Qwen2-0.5B gate|up at m = 64, 152 tiles: seven blocks per wave with
     // four waves, three or four with eight.)
     const size_t kMaxWaves =
+        max_waves ? max_waves :
         MT * NT > 2 && tiles > static_cast<size_t>(ctx->num_cus) ? (16 / (MT * NT) < 8 ? 16 / (MT * NT) : 8) : 8;
     size_t splits = 1;
-    if (tiles < static_cast<size_t>(ctx->num_cus) / 2) splits = (kb + kMaxWaves * BPW - 1) / (kMaxWaves * BPW);
+    if (rows * tiles < static_cast<size_t>(ctx->num_cus) / 2) splits = (kb + kMaxWaves * BPW - 1) / (kMaxWaves * BPW);
     if (splits > static_cast<size_t>(kMaxSplits)) splits = kMaxSplits;
     const size_t bps = (kb + splits - 1) / splits;
     splits = (kb + bps - 1) / bps;  // no empty split
@@ -1589,21 +1564,21 @@ int launch_skinny_t(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, con
     unsigned* counters = nullptr;
     const fh_edge ed = edge ? *edge : fh_edge{};
     if (splits > 1) {
-        const size_t part_bytes = splits * tiles * MT * NT * 1024 * sizeof(float);
+        const size_t part_bytes = rows * splits * tiles * MT * NT * 1024 * sizeof(float);
         if (scratch) {
             // The caller's fixed scratch: partials, then the arrival counters,
             // which are cleared here (a kernel, not a memset, so the call can
             // be captured into a graph).
             const size_t cnt_at = fh_align256(part_bytes);
-            if (cnt_at + tiles * sizeof(unsigned) > scratch->bytes)
+            if (cnt_at + rows * tiles * sizeof(unsigned) > scratch->bytes)
                 return fh_fail(ctx, FH_ERR_LIMIT,
                                "fh_q8_0_linear_noalloc: this shape needs " +
-                                   std::to_string(cnt_at + tiles * sizeof(unsigned)) +
+                                   std::to_string(cnt_at + rows * tiles * sizeof(unsigned)) +
                                    " bytes of scratch, above the fixed " + std::to_string(scratch->bytes));
             part = static_cast<float*>(scratch->ptr);
             counters = reinterpret_cast<unsigned*>(static_cast<char*>(scratch->ptr) + cnt_at);
-            hipLaunchKernelGGL(k_zero_counters, dim3(static_cast<unsigned>((tiles + 255) / 256)), dim3(256), 0,
-                               ctx->stream, counters, static_cast<int>(tiles));
+            hipLaunchKernelGGL(k_zero_counters, dim3(static_cast<unsigned>((rows * tiles + 255) / 256)), dim3(256),
+                               0, ctx->stream, counters, static_cast<int>(rows * tiles));
             FH_HIP(ctx, hipGetLastError());
         } else {
             void* ws = nullptr;
@@ -1611,13 +1586,13 @@ int launch_skinny_t(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, con
             if (rc) return rc;
             part = static_cast<float*>(ws);
             void* cnt = nullptr;
-            rc = fh_counter_area(ctx, tiles * sizeof(unsigned), &cnt);
+            rc = fh_counter_area(ctx, rows * tiles * sizeof(unsigned), &cnt);
             if (rc) return rc;
             counters = static_cast<unsigned*>(cnt);
         }
     }
     if (tiles > 0x7FFFFFFFu) return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: too many output columns");
-    const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(splits)), block(static_cast<unsigned>(64 * kw));
+    const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(splits), static_cast<unsigned>(rows)), block(static_cast<unsigned>(64 * kw));
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, block, lds, ctx->stream, x, w->qs, w->d, w->rexp, bias, y, static_cast<int>(m),
                            static_cast<int>(w->n), static_cast<int>(w->k), static_cast<int>(bps), part, counters, act,
@@ -1787,18 +1762,37 @@ int fh_launch_skinny_scratch(fh_ctx* ctx, const fh_q8_0* w, const float* x, size
     return launch_skinny(ctx, w, x, m, bias, y, &scratch);
 }
 
-// Tile choice: m <= 64 takes the skinny kernel; otherwise the 256 x 256
-// block-scaled tile (eight waves) once it still yields a tile per CU, the 128 x 128 tile at two
-// tiles per CU, else 64 x 64, else 32 x 32 outputs with four waves splitting K.
+// m <= 64 takes the skinny kernel.  Larger m takes the kernel and tile with the
+// least estimated time.  Fitted to timings over the GPT-2 and Qwen2-0.5B shapes
+// at m = 65 .. 16352 (256 CUs), with kb blocks of K:
+//  - the skinny kernel in row tiles of 32 (one 32 x 32 tile per workgroup, its
+//    waves splitting K: every load of a tile out at once): 4 us + kb * 0.42 ns per
+//    tile with four waves; with eight waves while two workgroups per CU hold all
+//    tiles;
+//  - the same in tiles of 64 x 64 (an activation block is split for 64 columns):
+//    5 us + kb * 620 ns per round of two workgroups per CU;
+//  - 128 x 128 tiles over the pre-split panel: 5 us + kb * 1730 ns per such round;
+//  - 256 x 256 tiles (k_gemm_bscale): 8 us + kb * 2500 ns per round of one per CU.
+// us, before (32 x 32, 64 x 64 or 128 x 128 panel tiles, or 256 x 256, by tile counts;
+// GELU as a kernel of its own up to 128 x 128) and now: 3072 x 768 with GELU at m =
+// 127 16.9 -> 8.0, 768 x 3072 at m = 511 37.8 -> 24.8, 2304 x 768 at m = 1024 46.8
+// -> 25.0, 1024 x 4096 at m = 2048 116 -> 77.
 int fh_launch_gemm_w8a32(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const float* bias, float* y,
                          int act) {
-    const size_t cus = static_cast<size_t>(ctx->num_cus);
-    if (m <= 64) return launch_skinny(ctx, w, x, m, bias, y, nullptr, act);  // GELU in its epilogue
-    int rc;
-    if (((m + 255) / 256) * ((w->n + 255) / 256) >= cus)
-        return launch_bscale(ctx, w, x, m, bias, y, act);  // GELU in its epilogue
-    else if (((m + 127) / 128) * ((w->n + 127) / 128) >= 2 * cus) rc = launch_gemm<128, 128, 2, 2, 1>(ctx, w, x, m, bias, y);
-    else if (((m + 63) / 64) * ((w->n + 63) / 64) >= 2 * cus) rc = launch_gemm<64, 64, 2, 2, 1>(ctx, w, x, m, bias, y);
-    else rc = launch_gemm<32, 32, 1, 1, 4>(ctx, w, x, m, bias, y);
-    return rc == FH_OK && act == FH_ACT_GELU ? fh_launch_gelu(ctx, y, m * w->n) : rc;
+    if (m <= 64) return launch_skinny(ctx, w, x, m, bias, y, nullptr, act);
+    const size_t cus = static_cast<size_t>(ctx->num_cus), kb = w->k / 32;
+    auto tiles = [&](size_t t) { return (m + t - 1) / t * ((w->n + t - 1) / t); };
+    auto rounds = [](size_t n, size_t per) { return (n + per - 1) / per; };
+    const size_t t32 = tiles(32), ns32 = 4000 + kb * t32 * 42 / 100, ns64 = 5000 + kb * 620 * rounds(tiles(64), 2 * cus);
+    const size_t ns128 = 5000 + kb * 1730 * rounds(tiles(128), 2 * cus);
+    const size_t ns256 = 8000 + kb * 2500 * rounds(tiles(256), cus);
+    const size_t rows = (m + 31) / 32;  // (grid.z)
+    const size_t skinny = t32 <= 2 * cus ? 0 : ns32 < ns64 ? ns32 : ns64, big = ns128 < ns256 ? ns128 : ns256;
+    if (skinny <= big && rows <= 65535) {
+        if (t32 <= 2 * cus) return launch_skinny_t<1, 1, 1>(ctx, w, x, m, bias, y, nullptr, act);
+        if (ns32 < ns64) return launch_skinny_t<1, 1, 1>(ctx, w, x, m, bias, y, nullptr, act, nullptr, kSkinnyPlain, 4);
+        return launch_skinny_t<2, 2, 1>(ctx, w, x, m, bias, y, nullptr, act, nullptr, kSkinnyPlain, 4);
+    }
+    return ns128 < ns256 ? launch_gemm<128, 128, 2, 2>(ctx, w, x, m, bias, y, act)
+                         : launch_bscale(ctx, w, x, m, bias, y, act);
 }

@@ -703,3 +703,42 @@ def test_w8a8_pairs_of_blocks_are_bit_exact(fh, orc, m, n, k):
         [0, 31, 32, 63, 64, m // 2, 255 % m, 256 % m, m - 2, m - 1]
     ref = orc.q8_0_linear_w8a8(x[rows], raw, n, b)
     assert np.array_equal(got[rows], ref, equal_nan=True)
+
+
+# Every kernel that 65 rows or more can take (fh_launch_gemm_w8a32): row tiles
+# of the skinny kernel with eight waves, with K split over workgroups (each row
+# tile its own partials and counters, twice in a row) and with four waves, its
+# 64 x 64 tiles, the 128 x 128 tile and the 256 x 256 one; ragged rows and
+# columns, a weight row with a non-finite scale, non-finite activations, GELU.
+@pytest.mark.parametrize("m,n,k", [(65, 33, 2048), (97, 700, 768), (127, 4065, 96), (130, 6100, 64), (511, 4090, 256),
+                                   (2049, 4001, 256), (4090, 4097, 96)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_prompt_rows_on_every_tile(fh, orc, m, n, k, gelu):
+    import torch
+
+    import ferrum_hip
+
+    raw = weight(orc, n, k, m + n + k)
+    raw.reshape(n, k // 32, 34)[n // 2, 0, :2] = np.array([np.inf], np.float16).view(np.uint8)
+    x, b = acts(m, k, m + 1), bias_for(n, k)
+    x[m // 2, k - 1], x[m - 1, 0] = np.inf, np.nan
+    w = ferrum_hip.Q8_0Weight.upload(fh, raw, n, k)
+    dx, db = torch.from_numpy(x).cuda(), torch.from_numpy(b).cuda()
+    dy = torch.full((2, m, n), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    for y in dy:
+        ferrum_hip.linear_act_async(fh, w, dx, m, k, db, n, y, ferrum_hip.ACT_GELU if gelu else ferrum_hip.ACT_NONE)
+    fh.sync()
+    got, again = dy.cpu().numpy()
+    w.free()
+    assert np.array_equal(got, again, equal_nan=True)
+    rows = np.unique(np.r_[sample_rows(m, 12, 3), 31, 32, 63, 64, m // 2])
+    want = orc.q8_0_linear(x[rows], raw, n, b)
+    finite = np.isfinite(want)
+    assert finite.any() and not finite.all()
+    with np.errstate(invalid="ignore"):
+        mass = np.where(finite, term_mass(orc, x[rows], raw, n, k), 0)
+        if gelu:
+            want, mass = orc.gelu(want), 1.13 * mass  # |gelu'| <= 1.13 carries the linear's bound over
+        assert np.array_equal(np.isnan(got[rows]), np.isnan(want))
+        assert_close(np.where(finite, got[rows], 0), np.where(finite, want, 0), mass)
