@@ -9,15 +9,16 @@
 // before the block come from the caches, the block's own from its q|k|v rows;
 // the same launch writes the block's k / v rows into the caches.
 //
-// How (head width 64): one workgroup per (128 query rows, head, sequence).
+// How (head widths 32 and 64): one workgroup per (128 query rows, head, sequence).
 // Each of its four waves owns 32 query rows and walks 32-key tiles of the
 // sequence's cache up to its last row's position; the tiles are staged in LDS
 // once for the four waves (double-buffered, the next tile's loads in flight
 // while the current one is used).  Per tile, flash style: S^T = K Q^T on the
 // matrix cores, the masked softmax with a running max and sum per query
 // (exact rescaling between tiles), then O += P V on the matrix cores, P
-// going in straight from the S^T accumulators and the outputs coming out one
-// query row per accumulator (coalesced stores).  The f32 operands ride on the
+// going in straight from the S^T accumulators as the B operand of O^T += V^T P^T,
+// so that a lane keeps to one query throughout: the rescaling and the final
+// division are by its own factors.  The f32 operands ride on the
 // f16 matrix cores as two terms each (k_attn_prefill_f16 below).
 #include "fh_internal.hpp"
 
@@ -27,10 +28,9 @@ namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kPT = 256;       // threads: four waves of 32 query rows
-constexpr int kQRows = 128;    // query rows per workgroup
 constexpr int kKeys = 32;      // keys per tile
-constexpr int kHd = 64;        // head width
+constexpr int kRT = 4;         // waves of 32 query rows that share a key tile
+constexpr int kPT = 64 * kRT, kQRows = 32 * kRT;
 
 struct PrefillArgs {
     const float* qkv;   // row s * rows + r; head h's q at column h * 64
@@ -39,7 +39,7 @@ struct PrefillArgs {
     float* vc;
     size_t seq_stride;
     int kv_dim;
-    int rows, pos0, groups;
+    int rows, pos0, groups, heads, pairs;  // groups of kQRows query rows; pairs = heads x sequences
     float scale;
     float* out;         // row s * rows + r; head h at column h * 64
     int out_ld;
@@ -55,22 +55,26 @@ __device__ __forceinline__ int acc_row(int v, int half) { return (v >> 2) * 8 + 
 // (the dropped l l' is 2^-22 of it), summed in f32 by v_mfma_f32_32x32x16_f16:
 // 12 MFMAs per 32-key tile for S^T = K Q^T and 12 for O += P V, against 32 +
 // 32 v_mfma_f32_32x32x2_f32 on the fp32 path, each of which takes twice an
-// f16 one's cycles (measured on the configs[3] prime: 10.6 -> 6.8 ms).
+// f16 one's cycles (32 prompts of 511 rows, 24 blocks: 10.6 -> 6.8 ms).
 //   q, k: each query row and each key row is scaled by its own power of two
 //     (its largest finite |value| into [2^14, 2^15)) before the split, and
-//     the score is unscaled exactly afterwards with the 1/sqrt(64) of the
-//     reference: s = S' * 2^-eq * 2^-ek / 8.  Non-finite values keep l = 0,
+//     the score is unscaled exactly afterwards with the 1/sqrt(hd) of the
+//     reference: s = S' * (2^-eq / sqrt(hd)) * 2^-ek.  Non-finite values keep l = 0,
 //     so inf and NaN reach the score as the f32 product gives them.
 //   P V: P (in [0, 1]) is split as it leaves the score accumulators; a lane's
-//     16 keys of its query are the A operand's two K16 steps as they stand
+//     16 keys of its query are the B operand's two K16 steps as they stand
 //     (keys 8 a + 4 half + (0..3)), and the v tile is staged transposed,
-//     [dim][key] with the keys in that same order, as the B operand.  A tile
+//     [dim][key] with the keys in that same order, as the A operand.  A tile
 //     whose v values are not all finite and below 2^15 in magnitude is
 //     finished on the vector units with only the attended keys (0 * inf would
 //     otherwise turn a masked key's v into NaN), v read from the cache.
 // The error is that of the 22-bit operands, ~2^-22 relative per product,
 // well inside the 1e-5 rule.
-constexpr int kHPitch = kHd + 8;   // K tile row pitch (halves): 144-byte rows
+// Bound: a wave's chain per tile, some 400 vector instructions, 24 dependent
+// MFMAs and the waits for LDS and the barrier (a tile of its own keys: 790 vector
+// instructions, shuffles through LDS for every row maximum and an LDS round trip
+// for the rescaling before).  32 prompts of 511 rows, 12 heads: 176 -> 106 us, of
+// which the order of the row groups (see the kernel) 40.
 constexpr int kVPitch = kKeys + 8;  // V tile (transposed) row pitch (halves): 80-byte rows
 
 typedef _Float16 h8f __attribute__((ext_vector_type(8)));
@@ -104,44 +108,95 @@ __device__ __forceinline__ float pow2f(int e) { return __builtin_bit_cast(float,
 // weight in a softmax, far inside the 1e-5 rule; -inf gives 0, NaN stays NaN.
 __device__ __forceinline__ float exp_approx(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 
-// Two scaled f32 values as f16 h and l terms (l = 0 for a non-finite value).
+typedef float f2f __attribute__((ext_vector_type(2)));
+
+// Two scaled f32 values as f16 h and l terms (SAFE: l = 0 for a non-finite value).
+template <bool SAFE>
 __device__ __forceinline__ void split2(float x0, float x1, float sc, h2f& h, h2f& l) {
-    const float s0 = x0 * sc, s1 = x1 * sc;
-    h = h2f{static_cast<_Float16>(s0), static_cast<_Float16>(s1)};
-    const float r0 = __builtin_isfinite(s0) ? s0 - static_cast<float>(h.x) : 0.0f;
-    const float r1 = __builtin_isfinite(s1) ? s1 - static_cast<float>(h.y) : 0.0f;
-    l = h2f{static_cast<_Float16>(r0), static_cast<_Float16>(r1)};
+    const f2f s = {x0 * sc, x1 * sc};
+    h = __builtin_convertvector(s, h2f);
+    f2f r = {s.x - static_cast<float>(h.x), s.y - static_cast<float>(h.y)};
+    if (SAFE) {
+        r.x = __builtin_isfinite(s.x) ? r.x : 0.0f;
+        r.y = __builtin_isfinite(s.y) ? r.y : 0.0f;
+    }
+    l = __builtin_convertvector(r, h2f);
 }
 
-__global__ void __launch_bounds__(kPT, 2) k_attn_prefill_f16(PrefillArgs a) {
-    __shared__ __align__(16) _Float16 kh[2][kKeys * kHPitch], kl[2][kKeys * kHPitch];
-    __shared__ __align__(16) _Float16 vh[2][kHd * kVPitch], vl[2][kHd * kVPitch];
-    __shared__ __align__(16) float kinv[2][kKeys];           // 2^-ek per key row
-    __shared__ __align__(16) float cx[4][32];                // per wave: one factor per query row
-    __shared__ __align__(16) float pt[4][kKeys * 33];        // per wave: P of a tile with unsafe v ([key][query])
+// Lane l's and lane l ^ 32's values, on the vector units (a shuffle goes through LDS).
+__device__ __forceinline__ float max_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), false, false);
+    return fmaxf(__builtin_bit_cast(float, static_cast<int>(r[0])), __builtin_bit_cast(float, static_cast<int>(r[1])));
+}
+// The largest value of each group of N = 8 or 16 lanes (xor 1, xor 2, half mirror, mirror), by
+// DPP operands.
+template <int CTRL>
+__device__ __forceinline__ float dpp_of(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+template <int N>
+__device__ __forceinline__ float max_row(float v) {
+    v = fmaxf(v, dpp_of<0xB1>(v));
+    v = fmaxf(v, dpp_of<0x4E>(v));
+    v = fmaxf(v, dpp_of<0x141>(v));
+    return N == 16 ? fmaxf(v, dpp_of<0x140>(v)) : v;
+}
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, half = lane >> 5, col = lane & 31;
-    const int g = a.groups - 1 - static_cast<int>(blockIdx.x);  // the longest rows first
-    const int h = blockIdx.y, s = blockIdx.z;
+// HD: the head width, 32 or 64.  HALVES = 2: eight waves, the first four on the
+// even key tiles and the others on the odd ones of the same 128 query rows, their
+// sums merged at the end (a wave's walk over its tiles is a chain: half as long,
+// where there are too few workgroups to fill the waves' waits with one another's
+// work).
+template <int HD, int HALVES>
+__global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs a) {
+    constexpr int kHPitch = HD + 8;          // K tile row pitch (halves): 16-byte pieces of 8 rows on different banks
+    constexpr int R4 = HD / 4;               // threads (float4s) per key row
+    constexpr int NK = kKeys * R4 / kPT;     // float4s of k per thread and tile
+    constexpr int KI = HD / 16, OT = HD / 32;  // MFMA K steps of a score, 32-dim output tiles
+    // one key tile, and per wave the P of a tile with unsafe v ([key][query])
+    struct Stage {
+        __align__(16) _Float16 kh[2][kKeys * kHPitch], kl[2][kKeys * kHPitch];
+        __align__(16) _Float16 vh[2][HD * kVPitch], vl[2][HD * kVPitch];
+        __align__(16) float kinv[2][kKeys];  // 2^-ek per key row
+        __align__(16) float pt[kRT][kKeys * 33];
+        int unsafe[3];                       // a tile's v is not safe for the split (step st: st % 3)
+    };
+    __shared__ Stage stages[HALVES];
+    static_assert(HALVES == 1 || sizeof(Stage) >= kRT * (2 + 16 * OT) * 64 * sizeof(float), "the merge fits a stage");
+    const int hf = HALVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kPT);
+    Stage& sm = stages[hf];
+    auto& kh = sm.kh;
+    auto& kl = sm.kl;
+    auto& vh = sm.vh;
+    auto& vl = sm.vl;
+    auto& kinv = sm.kinv;
+
+    const int tid = threadIdx.x % kPT, lane = tid & 63, half = lane >> 5, col = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // The longest rows of every head and sequence first.  (With a head's row
+    // groups next to each other, a group count of four or eight gave each XCD
+    // groups of one length, since workgroups are dealt to the eight in turn.)
+    const int g = a.groups - 1 - static_cast<int>(blockIdx.x) / a.pairs, pair = static_cast<int>(blockIdx.x) % a.pairs;
+    const int h = pair % a.heads, s = pair / a.heads;
     const int r0 = g * kQRows + wave * 32;
     const int last_row = min(a.rows - 1, g * kQRows + kQRows - 1);
     const int kmax = a.pos0 + last_row;
     const int ntiles = kmax / kKeys + 1;
     const int my_tiles = r0 < a.rows ? (a.pos0 + min(a.rows - 1, r0 + 31)) / kKeys + 1 : 0;
-    const size_t sbase = static_cast<size_t>(s) * a.seq_stride + static_cast<size_t>(h) * kHd;
+    const size_t sbase = static_cast<size_t>(s) * a.seq_stride + static_cast<size_t>(h) * HD;
     float* kc = a.kc + sbase;
     float* vc = a.vc + sbase;
 
-    // This lane's query: dims 16 i + 8 half + (0..7), i = 0..3 (the B
+    // This lane's query: dims 16 i + 8 half + (0..7), i < HD / 16 (the B
     // operand of step i), scaled by the row's power of two and split.
-    h8f qh[4], ql[4];
+    h8f qh[KI], ql[KI];
     float qscale;
     {
         const int row = min(r0 + col, a.rows - 1);
-        const float* qp = a.qkv + (static_cast<size_t>(s) * a.rows + row) * a.ld + h * kHd + half * 8;
-        float qv[32];
+        const float* qp = a.qkv + (static_cast<size_t>(s) * a.rows + row) * a.ld + h * HD + half * 8;
+        float qv[8 * KI];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < KI; i++) {
             const float4 u = *reinterpret_cast<const float4*>(qp + 16 * i);
             const float4 w = *reinterpret_cast<const float4*>(qp + 16 * i + 4);
             qv[8 * i] = u.x; qv[8 * i + 1] = u.y; qv[8 * i + 2] = u.z; qv[8 * i + 3] = u.w;
@@ -149,117 +204,148 @@ __global__ void __launch_bounds__(kPT, 2) k_attn_prefill_f16(PrefillArgs a) {
         }
         float mx = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 32; i++)
+        for (int i = 0; i < 8 * KI; i++)
             if (__builtin_isfinite(qv[i])) mx = fmaxf(mx, fabsf(qv[i]));
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));  // the other half of the row
         const int eq = pow2_exponent(mx);
         const float sc = pow2f(eq);
-        qscale = pow2f(-eq) * a.scale;  // (a.scale = 1/8: the product stays exact)
+        qscale = pow2f(-eq) * a.scale;  // (a power of two: exact)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < KI; i++)
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
                 h2f hh, ll;
-                split2(qv[8 * i + j], qv[8 * i + j + 1], sc, hh, ll);
+                split2<true>(qv[8 * i + j], qv[8 * i + j + 1], sc, hh, ll);
                 qh[i][j] = hh.x; qh[i][j + 1] = hh.y;
                 ql[i][j] = ll.x; ql[i][j + 1] = ll.y;
             }
     }
     const int qpos = a.pos0 + r0 + col;
 
-    // Tile staging: thread t takes float4s t and t + 256 of the k and of the v
-    // rows (row idx / 16, dims 4 (idx % 16) ...); the 16 threads of a key row
+    // Tile staging: thread t takes float4s t, t + kPT, ... of the k rows (row idx /
+    // 16, dims 4 (idx % 16) ...); the 16 threads of a key row
     // are consecutive lanes, so its exponent is a 16-lane reduction.  Keys of
     // the block itself (pos0 on) come from its q|k|v rows, earlier ones from
-    // the cache; workgroup 0 of each (sequence, head), which walks every tile,
+    // the cache; the last row group's workgroup of each (sequence, head), which walks every tile,
     // also writes the block's k and v rows into the cache as it stages them
     // (no other workgroup of the launch reads those cache rows).
-    const bool writer = blockIdx.x == 0;
-    const float* bq = a.qkv + static_cast<size_t>(s) * a.rows * a.ld + h * kHd;  // this sequence's block rows
+    const bool writer = g == a.groups - 1;
+    const float* bq = a.qkv + static_cast<size_t>(s) * a.rows * a.ld + h * HD;  // this sequence's block rows
     // The v rows go by pairs instead: thread t takes keys 2 (t / 16) and
-    // 2 (t / 16) + 1, dims 4 (t % 16) ..., which sit side by side in the
+    // 2 (t / 16) + 1 (and so on kPT / 8 keys further), dims 4 (t % 16) ..., which sit side by side in the
     // transposed tile, so each dim is one 4-byte store per term.
-    float4 pk[2], pv[2];
+    float4 pk[NK], pv[2];
+    const bool v_mine = HD == 64 || tid < kPT / 2;  // (wave-uniform)
     auto key_row = [&](int key, int off, const float* cache) __attribute__((always_inline)) {
         return key >= a.pos0 ? bq + static_cast<size_t>(key - a.pos0) * a.ld + off
                              : cache + static_cast<size_t>(key) * a.kv_dim;
     };
+    const int c0 = tid % R4 * 4;
+    auto k_key = [&](int i) { return tid / R4 + i * (kPT / R4); };
+    auto v_key = [&](int i) { return 2 * (tid / R4) + i; };  // (v_mine)
+    const float* bk = bq + a.kv_dim + c0;
+    const float* bv = bq + 2 * a.kv_dim + c0;
     auto fetch = [&](int t) __attribute__((always_inline)) {
+        if (t * kKeys >= a.pos0) {  // (uniform) every key is the block's own
+            const int r = t * kKeys - a.pos0, last = kmax - a.pos0;
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int idx = tid + i * kPT, c4 = idx & 15;
-            const int key = min(t * kKeys + (idx >> 4), kmax);
-            const int vkey = min(t * kKeys + 2 * (tid >> 4) + i, kmax);
-            pk[i] = *reinterpret_cast<const float4*>(key_row(key, a.kv_dim, kc) + c4 * 4);
-            pv[i] = *reinterpret_cast<const float4*>(key_row(vkey, 2 * a.kv_dim, vc) + c4 * 4);
+            for (int i = 0; i < NK; i++)
+                pk[i] = *reinterpret_cast<const float4*>(bk + static_cast<size_t>(min(r + k_key(i), last)) * a.ld);
+            if (v_mine)
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    pv[i] = *reinterpret_cast<const float4*>(bv + static_cast<size_t>(min(r + v_key(i), last)) * a.ld);
+            return;
         }
+#pragma unroll
+        for (int i = 0; i < NK; i++)
+            pk[i] = *reinterpret_cast<const float4*>(key_row(min(t * kKeys + k_key(i), kmax), a.kv_dim, kc) + c0);
+        if (v_mine)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                pv[i] = *reinterpret_cast<const float4*>(key_row(min(t * kKeys + v_key(i), kmax), 2 * a.kv_dim, vc) + c0);
     };
     auto store_block_rows = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int idx = tid + i * kPT, c4 = idx & 15;
-            const int key = t * kKeys + (idx >> 4), vkey = t * kKeys + 2 * (tid >> 4) + i;
+        for (int i = 0; i < NK; i++) {
+            const int key = t * kKeys + k_key(i);
             if (key >= a.pos0 && key <= kmax)
-                *reinterpret_cast<float4*>(kc + static_cast<size_t>(key) * a.kv_dim + c4 * 4) = pk[i];
-            if (vkey >= a.pos0 && vkey <= kmax)
-                *reinterpret_cast<float4*>(vc + static_cast<size_t>(vkey) * a.kv_dim + c4 * 4) = pv[i];
+                *reinterpret_cast<float4*>(kc + static_cast<size_t>(key) * a.kv_dim + c0) = pk[i];
         }
-    };
-    // returns whether this thread's v values are unsafe for the f16 split
-    auto stash = [&](int buf) __attribute__((always_inline)) -> bool {
-        bool bad = false;
+        if (v_mine)
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const int idx = tid + i * kPT, row = idx >> 4, c0 = (idx & 15) * 4;
+            for (int i = 0; i < 2; i++) {
+                const int key = t * kKeys + v_key(i);
+                if (key >= a.pos0 && key <= kmax)
+                    *reinterpret_cast<float4*>(vc + static_cast<size_t>(key) * a.kv_dim + c0) = pv[i];
+            }
+    };
+    auto stash = [&](int st) __attribute__((always_inline)) {
+        const int buf = st & 1;
+#pragma unroll
+        for (int i = 0; i < NK; i++) {
+            const int row = k_key(i);
             const float4 k4 = pk[i];
-            float mx = 0.0f;
-            if (__builtin_isfinite(k4.x)) mx = fmaxf(mx, fabsf(k4.x));
-            if (__builtin_isfinite(k4.y)) mx = fmaxf(mx, fabsf(k4.y));
-            if (__builtin_isfinite(k4.z)) mx = fmaxf(mx, fabsf(k4.z));
-            if (__builtin_isfinite(k4.w)) mx = fmaxf(mx, fabsf(k4.w));
-            mx = fmaxf(mx, __shfl_xor(mx, 1, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 2, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 4, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 8, 64));
-            const int ek = pow2_exponent(mx);
+            // fmaxf skips NaN (whose terms are NaN without a guard, as its
+            // score is); an infinite maximum takes the rare guarded path.
+            float mx = max_row<R4>(fmaxf(fmaxf(fabsf(k4.x), fabsf(k4.y)), fmaxf(fabsf(k4.z), fabsf(k4.w))));
+            int ek;
             h2f h01, l01, h23, l23;
-            split2(k4.x, k4.y, pow2f(ek), h01, l01);
-            split2(k4.z, k4.w, pow2f(ek), h23, l23);
+            if (__builtin_expect(__ballot(!__builtin_isfinite(mx)) != 0, 0)) {
+                float fm = 0.0f;
+                if (__builtin_isfinite(k4.x)) fm = fmaxf(fm, fabsf(k4.x));
+                if (__builtin_isfinite(k4.y)) fm = fmaxf(fm, fabsf(k4.y));
+                if (__builtin_isfinite(k4.z)) fm = fmaxf(fm, fabsf(k4.z));
+                if (__builtin_isfinite(k4.w)) fm = fmaxf(fm, fabsf(k4.w));
+                ek = pow2_exponent(max_row<R4>(fm));
+                split2<true>(k4.x, k4.y, pow2f(ek), h01, l01);
+                split2<true>(k4.z, k4.w, pow2f(ek), h23, l23);
+            } else {
+                ek = pow2_exponent(mx);
+                split2<false>(k4.x, k4.y, pow2f(ek), h01, l01);
+                split2<false>(k4.z, k4.w, pow2f(ek), h23, l23);
+            }
             *reinterpret_cast<uint2*>(&kh[buf][row * kHPitch + c0]) =
                 make_uint2(__builtin_bit_cast(uint32_t, h01), __builtin_bit_cast(uint32_t, h23));
             *reinterpret_cast<uint2*>(&kl[buf][row * kHPitch + c0]) =
                 make_uint2(__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23));
             if (c0 == 0) kinv[buf][row] = pow2f(-ek);
         }
-        const int c0 = (tid & 15) * 4, kp = vkey_pos(2 * (tid >> 4));  // even; the pair's second key at kp + 1
+        if (!v_mine) return;
+        const int kp = vkey_pos(v_key(0));  // even; the pair's second key at kp + 1
         const float va[4] = {pv[0].x, pv[0].y, pv[0].z, pv[0].w};
         const float vb[4] = {pv[1].x, pv[1].y, pv[1].z, pv[1].w};
+        uint32_t top = 0;  // the largest magnitude's bits (inf and NaN above every finite one)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            bad |= !(fabsf(va[j]) < 32768.0f) || !(fabsf(vb[j]) < 32768.0f);  // (also NaN)
-            const h2f hv = h2f{static_cast<_Float16>(va[j]), static_cast<_Float16>(vb[j])};
-            const h2f lv = h2f{static_cast<_Float16>(va[j] - static_cast<float>(hv.x)),
-                               static_cast<_Float16>(vb[j] - static_cast<float>(hv.y))};
+            top = max(top, max(__builtin_bit_cast(uint32_t, va[j]) & 0x7FFFFFFFu,
+                               __builtin_bit_cast(uint32_t, vb[j]) & 0x7FFFFFFFu));
+            h2f hv, lv;
+            split2<false>(va[j], vb[j], 1.0f, hv, lv);
             const int at = vt_pos(c0 + j, kp);
             *reinterpret_cast<uint32_t*>(&vh[buf][at]) = __builtin_bit_cast(uint32_t, hv);
             *reinterpret_cast<uint32_t*>(&vl[buf][at]) = __builtin_bit_cast(uint32_t, lv);
         }
-        return bad;
+        if (__builtin_expect(top >= 0x47000000u, 0)) sm.unsafe[st % 3] = 1;  // 2^15 or more
     };
 
     float m_run = -INFINITY, l_run = 0.0f;
-    f32x16 o0, o1;
+    f32x16 o[OT];
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        o0[v] = 0.0f;
-        o1[v] = 0.0f;
-    }
-    fetch(0);
-    if (writer) store_block_rows(0);
-    bool vbad = __syncthreads_or(stash(0));
-    for (int t = 0; t < ntiles; t++) {
-        const int buf = t & 1, k0 = t * kKeys;
-        if (t + 1 < ntiles) fetch(t + 1);
+    for (int d = 0; d < OT; d++) o[d] = f32x16{};
+    // this half's tiles: hf, hf + HALVES, ... (a step past ntiles stages nothing)
+    const int steps = (ntiles + HALVES - 1) / HALVES;
+    if (tid < 3) sm.unsafe[tid] = 0;
+    fetch(hf);
+    if (writer) store_block_rows(hf);
+    __syncthreads();
+    stash(0);
+    __syncthreads();
+    for (int st = 0; st < steps; st++) {
+        const int t = st * HALVES + hf, tn = t + HALVES, buf = st & 1, k0 = t * kKeys;
+        if (tn < ntiles) fetch(tn);
+        const bool vbad = sm.unsafe[st % 3] != 0;
+        if (tid == 0) sm.unsafe[(st + 2) % 3] = 0;  // (read at step st - 1, written next at step st + 1)
         if (t < my_tiles) {
             // ---- S'^T = K Q^T (scaled terms): accumulator v of lane (half, col) is key acc_row(v, half), query col
             f32x16 sacc;
@@ -268,7 +354,7 @@ __global__ void __launch_bounds__(kPT, 2) k_attn_prefill_f16(PrefillArgs a) {
             const _Float16* khr = &kh[buf][col * kHPitch + half * 8];
             const _Float16* klr = &kl[buf][col * kHPitch + half * 8];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < KI; i++) {
                 const h8f a_h = *reinterpret_cast<const h8f*>(khr + 16 * i);
                 const h8f a_l = *reinterpret_cast<const h8f*>(klr + 16 * i);
                 sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_h, qh[i], sacc, 0, 0, 0);
@@ -276,6 +362,7 @@ __global__ void __launch_bounds__(kPT, 2) k_attn_prefill_f16(PrefillArgs a) {
                 sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(a_l, qh[i], sacc, 0, 0, 0);
             }
             // ---- scores, unscaled exactly, masked past the query's position
+            // (only the last tiles of a wave hold masked keys)
             float sv[16];
             float mt = -INFINITY;
 #pragma unroll
@@ -283,107 +370,111 @@ __global__ void __launch_bounds__(kPT, 2) k_attn_prefill_f16(PrefillArgs a) {
                 const float4 ki = *reinterpret_cast<const float4*>(&kinv[buf][a4 * 8 + half * 4]);
                 const float kv4[4] = {ki.x, ki.y, ki.z, ki.w};
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int v = 4 * a4 + j;
-                    sv[v] = k0 + acc_row(v, half) <= qpos ? sacc[v] * qscale * kv4[j] : -INFINITY;
-                    mt = fmaxf(mt, sv[v]);
-                }
+                for (int j = 0; j < 4; j++) sv[4 * a4 + j] = sacc[4 * a4 + j] * qscale * kv4[j];
             }
-            mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-            const float m_new = fmaxf(m_run, mt);
-            const float corr = exp_approx(m_run - m_new);  // 0 on the first tile (m_run = -inf)
+            if (k0 + kKeys - 1 > a.pos0 + r0)
+#pragma unroll
+                for (int v = 0; v < 16; v++) sv[v] = k0 + acc_row(v, half) <= qpos ? sv[v] : -INFINITY;
+#pragma unroll
+            for (int v = 0; v < 16; v++) mt = fmaxf(mt, sv[v]);
+            // (a query whose scores so far are all -inf, masked ones among them,
+            // keeps sums of 0, and 0 / 0 = NaN if it ends so)
+            const float m_new = fmaxf(m_run, max_halves(mt)), m_exp = m_new == -INFINITY ? 0.0f : m_new;
+            const float corr = exp_approx(m_run - m_exp);  // 0 on the first tile (m_run = -inf)
             float ps = 0.0f;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                sv[v] = exp_approx(sv[v] - m_new);
+                sv[v] = exp_approx(sv[v] - m_exp);
                 ps += sv[v];
             }
-            ps += __shfl_xor(ps, 32, 64);
-            l_run = l_run * corr + ps;
+            l_run = l_run * corr + ps;  // (this half's keys; the halves are added at the end)
             m_run = m_new;
-            if (half == 0) cx[wave][col] = corr;
-            __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int a4 = 0; a4 < 4; a4++) {
-                const float4 c = *reinterpret_cast<const float4*>(&cx[wave][a4 * 8 + half * 4]);
-                o0[4 * a4] *= c.x;
-                o0[4 * a4 + 1] *= c.y;
-                o0[4 * a4 + 2] *= c.z;
-                o0[4 * a4 + 3] *= c.w;
-                o1[4 * a4] *= c.x;
-                o1[4 * a4 + 1] *= c.y;
-                o1[4 * a4 + 2] *= c.z;
-                o1[4 * a4 + 3] *= c.w;
-            }
-            __builtin_amdgcn_wave_barrier();
+            for (int d = 0; d < OT; d++) o[d] *= corr;
             if (!vbad) {
-                // ---- O += P V: step st takes this lane's keys acc_row(8 st + j, half)
+                // ---- O^T += V^T P^T: step s2 takes this lane's keys acc_row(8 s2 + j, half)
 #pragma unroll
-                for (int st = 0; st < 2; st++) {
+                for (int s2 = 0; s2 < 2; s2++) {
                     h8f ph, pl;
 #pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        const float p = sv[8 * st + j];
-                        ph[j] = static_cast<_Float16>(p);
-                        pl[j] = static_cast<_Float16>(p - static_cast<float>(ph[j]));
+                    for (int j = 0; j < 8; j += 2) {
+                        h2f hh, ll;
+                        split2<false>(sv[8 * s2 + j], sv[8 * s2 + j + 1], 1.0f, hh, ll);
+                        ph[j] = hh.x; ph[j + 1] = hh.y;
+                        pl[j] = ll.x; pl[j + 1] = ll.y;
                     }
-                    const int off = 16 * st + 8 * half, at0 = vt_pos(col, off), at1 = vt_pos(32 + col, off);
-                    const h8f v0h = *reinterpret_cast<const h8f*>(&vh[buf][at0]);
-                    const h8f v0l = *reinterpret_cast<const h8f*>(&vl[buf][at0]);
-                    const h8f v1h = *reinterpret_cast<const h8f*>(&vh[buf][at1]);
-                    const h8f v1l = *reinterpret_cast<const h8f*>(&vl[buf][at1]);
-                    o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ph, v0h, o0, 0, 0, 0);
-                    o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ph, v0l, o0, 0, 0, 0);
-                    o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pl, v0h, o0, 0, 0, 0);
-                    o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ph, v1h, o1, 0, 0, 0);
-                    o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(ph, v1l, o1, 0, 0, 0);
-                    o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(pl, v1h, o1, 0, 0, 0);
+                    const int off = 16 * s2 + 8 * half;
+                    h8f v_h[OT], v_l[OT];
+#pragma unroll
+                    for (int d = 0; d < OT; d++) {
+                        v_h[d] = *reinterpret_cast<const h8f*>(&vh[buf][vt_pos(32 * d + col, off)]);
+                        v_l[d] = *reinterpret_cast<const h8f*>(&vl[buf][vt_pos(32 * d + col, off)]);
+                    }
+#pragma unroll
+                    for (int d = 0; d < OT; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_h[d], ph, o[d], 0, 0, 0);
+#pragma unroll
+                    for (int d = 0; d < OT; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_l[d], ph, o[d], 0, 0, 0);
+#pragma unroll
+                    for (int d = 0; d < OT; d++) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v_h[d], pl, o[d], 0, 0, 0);
                 }
             } else {
                 // ---- v not safe for the split: only the attended keys, on the vector units
-                float* pw = pt[wave];
+                float* pw = sm.pt[wave];
 #pragma unroll
                 for (int v = 0; v < 16; v++) pw[acc_row(v, half) * 33 + col] = sv[v];
                 __builtin_amdgcn_wave_barrier();
+                for (int kk = 0; kk < kKeys && k0 + kk <= qpos; kk++) {
+                    const float p = pw[kk * 33 + col];
+                    const float* vrow = key_row(k0 + kk, 2 * a.kv_dim, vc);
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int qr = acc_row(v, half), qp = a.pos0 + r0 + qr;
-                    float s0 = o0[v], s1 = o1[v];
-                    for (int kk = 0; kk < kKeys && k0 + kk <= qp; kk++) {
-                        const float p = pw[kk * 33 + qr];
-                        const int key = k0 + kk;
-                        const float* vrow = key_row(key, 2 * a.kv_dim, vc);
-                        s0 += p * vrow[col];
-                        s1 += p * vrow[32 + col];
-                    }
-                    o0[v] = s0;
-                    o1[v] = s1;
+                    for (int d = 0; d < OT; d++)
+#pragma unroll
+                        for (int v = 0; v < 16; v++) o[d][v] += p * vrow[32 * d + acc_row(v, half)];
                 }
                 __builtin_amdgcn_wave_barrier();
             }
         }
-        bool vbad_next = false;
-        if (t + 1 < ntiles) {
-            if (writer) store_block_rows(t + 1);
-            vbad_next = stash(buf ^ 1);
+        if (tn < ntiles) {
+            if (writer) store_block_rows(tn);
+            stash(st + 1);
         }
-        vbad = __syncthreads_or(vbad_next);
+        __syncthreads();
+    }
+    float l = l_run + __shfl_xor(l_run, 32, 64);
+    if constexpr (HALVES == 2) {
+        // the odd tiles' maximum, sum and outputs through their stage's LDS
+        // (every wave is past its last read of it), scaled to the common maximum
+        float* mg = reinterpret_cast<float*>(&stages[1]) + wave * ((2 + 16 * OT) * 64) + lane;
+        if (hf == 1) {
+            mg[0] = m_run;
+            mg[64] = l;
+#pragma unroll
+            for (int d = 0; d < OT; d++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) mg[(2 + 16 * d + v) * 64] = o[d][v];
+        }
+        __syncthreads();
+        if (hf == 1) return;
+        const float m1 = mg[0], m = fmaxf(m_run, m1), m_exp = m == -INFINITY ? 0.0f : m;
+        const float f0 = exp_approx(m_run - m_exp), f1 = exp_approx(m1 - m_exp);
+        l = l * f0 + mg[64] * f1;
+#pragma unroll
+        for (int d = 0; d < OT; d++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) o[d][v] = o[d][v] * f0 + mg[(2 + 16 * d + v) * 64] * f1;
     }
 
-    // ---- out[row] = O / (sum of the row's exponentials)
-    if (r0 >= a.rows) return;
-    if (half == 0) cx[wave][col] = l_run;
-    __builtin_amdgcn_wave_barrier();
+    // ---- out[row] = O / (sum of the row's exponentials): lane (half, col) holds
+    // dims 8 a + 4 half + (0..3) of both 32-dim halves of query row col
+    const int row = r0 + col;
+    if (row >= a.rows) return;
+    float* op = a.out + (static_cast<size_t>(s) * a.rows + row) * a.out_ld + h * HD + half * 4;
 #pragma unroll
-    for (int v = 0; v < 16; v++) {
-        const int qr = acc_row(v, half), row = r0 + qr;
-        const float l = cx[wave][qr];
-        if (row < a.rows) {
-            float* op = a.out + (static_cast<size_t>(s) * a.rows + row) * a.out_ld + h * kHd;
-            op[col] = o0[v] / l;
-            op[32 + col] = o1[v] / l;
-        }
-    }
+    for (int d = 0; d < OT; d++)
+#pragma unroll
+        for (int a4 = 0; a4 < 4; a4++)
+            *reinterpret_cast<float4*>(op + 32 * d + 8 * a4) =
+                make_float4(o[d][4 * a4] / l, o[d][4 * a4 + 1] / l, o[d][4 * a4 + 2] / l, o[d][4 * a4 + 3] / l);
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -393,7 +484,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, float* vc, size_t seq_stride,
                                      size_t d, size_t heads, size_t pos0, size_t rows, size_t seqs, float* out) {
     const size_t hd = d / heads;
-    const bool mfma = hd == static_cast<size_t>(kHd) && aligned16(qkv) && aligned16(kc) && aligned16(vc) &&
+    const bool mfma = (hd == 32 || hd == 64) && aligned16(qkv) && aligned16(kc) && aligned16(vc) &&
                       aligned16(out) && seq_stride % 4 == 0;
     if (!mfma) {
         // other head widths: the vector-unit kernel, one sequence at a time
@@ -413,13 +504,31 @@ int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, f
     a.kv_dim = static_cast<int>(d);
     a.rows = static_cast<int>(rows);
     a.pos0 = static_cast<int>(pos0);
-    a.groups = static_cast<int>((rows + kQRows - 1) / kQRows);
     a.scale = 1.0f / sqrtf(static_cast<float>(hd));
     a.out = out;
     a.out_ld = static_cast<int>(d);
-    hipLaunchKernelGGL(k_attn_prefill_f16,
-                       dim3(static_cast<unsigned>(a.groups), static_cast<unsigned>(heads), static_cast<unsigned>(seqs)),
-                       dim3(kPT), 0, ctx->stream, a);
+    const size_t cus = static_cast<size_t>(ctx->num_cus), pairs = heads * seqs, groups = (rows + kQRows - 1) / kQRows;
+    if (pairs * groups > 0x7FFFFFFFu) return fh_fail(ctx, FH_ERR_LIMIT, "attention_prefill: too many heads and sequences");
+    a.heads = static_cast<int>(heads);
+    a.pairs = static_cast<int>(pairs);
+    a.groups = static_cast<int>(groups);
+    // One or two chains of key tiles per row.  Measured (ns, head width 64): a
+    // workgroup takes 2200 per tile alone on its CU, a CU of two 1750 per tile;
+    // with two chains 1500 alone (one workgroup per CU) and 2300, and 1500 for the
+    // merge.  8 sequences of 300 rows and 12 heads (288 workgroups of 4, 8 and 10
+    // tiles): 25.2 us and 22.5; 16 heads: 25.7 and 27.5; one of 511 rows: 33.4 and
+    // 25.6; 32 of 511: 106.8 and 131.4.
+    size_t tiles = 0;
+    for (size_t g = 1; g <= groups; g++) tiles += (pos0 + (g * kQRows < rows ? g * kQRows : rows) - 1) / kKeys + 1;
+    const size_t longest = (pos0 + rows - 1) / kKeys + 1, share = tiles * pairs / cus;
+    const size_t one = longest * 2200 > share * 1750 ? longest * 2200 : share * 1750;
+    const size_t two = (longest * 1500 > share * 2300 ? longest * 1500 : share * 2300) + 1500;
+    auto go = [&](auto kern, int halves) {
+        hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(pairs * groups)), dim3(static_cast<unsigned>(kPT * halves)), 0,
+                           ctx->stream, a);
+    };
+    if (hd == 64) two < one ? go(k_attn_prefill_f16<64, 2>, 2) : go(k_attn_prefill_f16<64, 1>, 1);
+    else two < one ? go(k_attn_prefill_f16<32, 2>, 2) : go(k_attn_prefill_f16<32, 1>, 1);
     FH_HIP(ctx, hipGetLastError());
     return FH_OK;
 }

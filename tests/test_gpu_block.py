@@ -745,3 +745,36 @@ def test_config1_greedy_run_on_the_device(fh, orc):
         assert checked >= 8
     finally:
         model.free()
+
+
+# The prompt attention's one and two chains of key tiles (by the launch's size)
+# at both head widths: rows and earlier positions on and beside the 32-key and
+# 128-row tiles (a row whose keys all lie in the even tiles, tiles that a query
+# does not reach), scores of -inf, and a tile whose v goes on the vector units.
+@pytest.mark.parametrize("d,heads", [(128, 2), (64, 2), (96, 3)])
+@pytest.mark.parametrize("seqs,rows,pos0", [(1, 1, 0), (1, 33, 31), (2, 65, 40), (1, 130, 0), (3, 129, 95), (260, 40, 1)])
+def test_prompt_attention_on_every_chain_and_width(fh, orc, d, heads, seqs, rows, pos0):
+    import ferrum_hip
+
+    cap = pos0 + rows
+    rng = np.random.default_rng(d + seqs + rows + pos0)
+    qkv = (rng.standard_normal((seqs * rows, 3 * d)) * 1.5).astype(np.float32)
+    kc, vc = (rng.standard_normal((seqs, cap, d)).astype(np.float32) for _ in range(2))
+    if pos0 > 2:  # keys whose scores overflow to -inf, and a large v
+        for h in range(heads):
+            qkv[:, h * (d // heads)] = 50.0
+            kc[:, 1:3, h * (d // heads)] = -3e38
+            kc[:, 3:, h * (d // heads)] = kc[:, 0, h * (d // heads)] = 0.125
+            qkv[:, d + h * (d // heads)] = 0.125
+        vc[0, 2, 5] = 1e6
+    tk, tv = dev(kc), dev(vc)
+    out = dev(np.zeros((seqs * rows, d), np.float32))
+    ready()
+    ferrum_hip.attention_prefill_seqs_async(fh, dev(qkv), tk, tv, cap * d, cap, d, heads, pos0, rows, seqs, out)
+    got = host(fh, out)
+    for s in {0, seqs // 2, seqs - 1}:
+        ko, vo = kc[s].copy(), vc[s].copy()
+        for r in range(rows):
+            want = orc.attention_decode(qkv[s * rows + r], ko, vo, heads, pos0 + r)
+            close(got[s * rows + r], want, 1e-5)
+        assert np.array_equal(host(fh, tk)[s], ko) and np.array_equal(host(fh, tv)[s], vo)
