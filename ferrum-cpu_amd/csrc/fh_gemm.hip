@@ -941,11 +941,16 @@ __global__ void __launch_bounds__(512)
     k_gemm_skinny(const float* __restrict__ x, const int8_t* __restrict__ qs, const uint16_t* __restrict__ dsc,
                   const int8_t* __restrict__ rexp, const float* __restrict__ bias, float* y, int m, int n,
                   int k, int bps, float* __restrict__ part, unsigned* __restrict__ counters, int act, fh_edge e) {
-    if constexpr (MODE == kSkinnyPlain) {  // grid.z: tiles of 32 MT rows (one in the other modes)
+    {  // grid.z: tiles of 32 MT rows
         const size_t rows = static_cast<size_t>(blockIdx.z) * (32 * MT);
         x += rows * k;
-        y += rows * n;
+        y += rows * (MODE == kSkinnyNormGlu ? n >> 1 : n);
         m -= static_cast<int>(rows);
+        if constexpr (MODE == kSkinnyNormIn || MODE == kSkinnyNormGlu) e.stats += rows * (k >> 5) * 2;
+        if constexpr (MODE == kSkinnyResOut) {
+            e.r += rows * n;
+            e.stats += rows * (n >> 5) * 2;
+        }
         part += static_cast<size_t>(blockIdx.z) * gridDim.y * gridDim.x * (MT * NT * 1024);
         counters += static_cast<size_t>(blockIdx.z) * gridDim.x;
     }
@@ -1645,11 +1650,14 @@ constexpr size_t kWideMinTiles = 1024;
 // Tile rules from timings at m = 32 and 64 over the GPT-2 and Qwen2-0.5B
 // shapes: two column tiles per wave pay off from about 256 tiles of 32
 // columns (a 9728-wide output: 14.2 -> 11.8 us at m = 32), four only at m <=
-// 32 (four at m = 64 ran the 151936-wide head 2.8x slower); at m = 64 two
-// blocks per wave batch beat three (small layers 11.4 -> 10.4 us); at m <=
-// 32 and 64 outputs narrower than 2048 take one block per wave batch (more K
-// splits, so more workgroups: 896 x 896 7.9 -> 6.9 us at m = 32, 10.4 -> 9.2
-// us at m = 64; a 3072-wide one slows down).
+// 32 (four at m = 64 ran the 151936-wide head 2.8x slower); outputs narrower
+// than 2048 take one block per wave batch (more K splits, so more workgroups:
+// 896 x 896 7.9 -> 6.9 us at m = 32; a 3072-wide one slows down).  Below 256 tiles
+// of 32 columns, 33 to 64 rows are two row tiles of workgroups rather than two
+// per wave: 2304 x 768 at m = 64 10.7 -> 6.2 us, 768 x 3072 9.9 -> 8.2, a GPT-2
+// block of 64 sequences 68.2 -> 51.1; from there on one 64-row pass over the
+// weight is as fast (9728 x 896: 13.4 us both ways) or faster (with SwiGLU: a Qwen2
+// block of 64 sequences 58.6 against 63.5).
 int launch_skinny(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const float* bias, float* y,
                   const fh_scratch* scratch = nullptr, int act = FH_ACT_NONE, const fh_edge* edge = nullptr,
                   int mode = kSkinnyPlain) {
@@ -1674,16 +1682,14 @@ int launch_skinny(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const
         return act == FH_ACT_GELU ? fh_launch_gelu(ctx, y, m * w->n) : FH_OK;
     }
     // (the fused edges never take the 4-group tiles: at t32 >= 1024 they take 2)
-    if (m <= 32) {
+    if (m <= 32 || t32 < 256) {
         if (t32 >= 4 * 256 && mode == kSkinnyPlain) return launch_skinny_t<1, 4, 2>(ctx, w, x, m, bias, y, scratch, act);
         if (t32 >= 256) return launch_skinny_t<1, 2, 3>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
         if (t32 >= 64) return launch_skinny_t<1, 1, 3>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
         return launch_skinny_t<1, 1, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
     }
     if (t32 >= 4 * 256 && mode == kSkinnyPlain) return launch_skinny_t<2, 2, 2>(ctx, w, x, m, bias, y, scratch, act);
-    if (t32 >= 256) return launch_skinny_t<2, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
-    if (t32 >= 64) return launch_skinny_t<2, 1, 2>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
-    return launch_skinny_t<2, 1, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);  // 896 x 896: 10.4 -> 9.2 us
+    return launch_skinny_t<2, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
 }
 
 }  // namespace

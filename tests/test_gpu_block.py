@@ -461,6 +461,48 @@ def test_linear_normed_matches_oracle(fh, orc, m, n, k, rms, act):
     w.free()
 
 
+@pytest.mark.parametrize("m,n,k", [(33, 640, 768), (45, 2304, 768), (63, 96, 3072), (64, 8160, 128), (64, 8192, 128),
+                                   (34, 32, 32)])
+def test_two_row_tiles_of_workgroups(fh, orc, m, n, k):
+    """33 to 64 rows of an output below 256 tiles of 32 columns (8192: one
+    64-row pass instead) are two row tiles of workgroups, the second ragged:
+    the normed-in and the residual-out linear against the oracle, and that the second tile's rows read and write their own
+    statistics."""
+    import torch
+
+    import ferrum_hip
+
+    rng = np.random.default_rng(m * 3 + n + k)
+    raw = orc.quantize_weight(n, k, n + 2 * k, 0.05)
+    w = ferrum_hip.Q8_0Weight.upload(fh, raw, n, k)
+    x = (rng.standard_normal((m, k)) * 2 + 0.5 * np.arange(m)[:, None] / m).astype(np.float32)
+    g = rng.standard_normal(k).astype(np.float32)
+    be = (rng.standard_normal(k) * 0.1).astype(np.float32)
+    b = (rng.standard_normal(n) * 0.1).astype(np.float32)
+    r = rng.standard_normal((m, n)).astype(np.float32)
+    y, z = torch.empty((m, n), device="cuda"), torch.empty((m, n), device="cuda")
+    st = dev(np.full((m, n // 32, 2), np.nan, np.float32))
+    ready()
+    ferrum_hip.linear_normed_async(fh, w, dev(x), m, k, dev(group_stats(x).astype(np.float32)), dev(g), dev(be), 1e-5,
+                                   False, dev(b), n, y, 0)
+    ferrum_hip.linear_residual_async(fh, w, dev(x), m, k, dev(b), n, dev(r), z, st)
+    # 1e-5 of the summed terms' magnitudes: the oracle's own f32 sum of k terms
+    # strays by up to k 2^-24 of them, 1.8e-4 at k = 3072, so 1e-5 of the
+    # result (which cancels to ~1/50 of its terms here) is below what it holds
+    h, wt = orc.layernorm(x, g, be), np.abs(orc.q8_0_to_ferrum_weight(raw, n, k).astype(np.float64))
+    lin = orc.q8_0_linear(h, raw, n, b)
+    mass = np.abs(h.astype(np.float64)) @ wt
+    assert (np.abs(host(fh, y).astype(np.float64) - lin) <= 1e-5 * np.maximum(np.abs(lin), mass)).all()
+    lin = orc.q8_0_linear(x, raw, n, b)
+    want, got = (r + lin).astype(np.float32), host(fh, z)
+    mass = np.abs(x.astype(np.float64)) @ wt
+    assert (np.abs(got.astype(np.float64) - want) <= 1e-5 * np.maximum(np.abs(lin), mass) + 6e-8 * np.abs(want)).all()
+    gs, ws = host(fh, st), group_stats(got)
+    np.testing.assert_allclose(gs[..., 0], ws[..., 0], rtol=1e-5, atol=1e-6 * np.abs(got).max())
+    np.testing.assert_allclose(gs[..., 1], ws[..., 1], rtol=2e-5)
+    w.free()
+
+
 @pytest.mark.parametrize("m,ffn,k,rms,bias", [(64, 4864, 896, True, False), (32, 4864, 896, True, False),
                                                (5, 256, 128, True, False), (40, 160, 1024, True, False),
                                                (3, 96, 64, False, True), (33, 4864, 896, False, True)])
