@@ -1662,9 +1662,12 @@ int launch_skinny(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const
                   const fh_scratch* scratch = nullptr, int act = FH_ACT_NONE, const fh_edge* edge = nullptr,
                   int mode = kSkinnyPlain) {
     const size_t t32 = (w->n + 31) / 32;
-    // the fused SwiGLU needs each workgroup's two column groups to be a gate / up pair
+    // the fused SwiGLU needs each workgroup's two column groups to be a gate / up
+    // pair; one Q8_0 block per wave batch (four batches of a 896-deep K per wave) beats
+    // two and three: a Qwen2 block of 3 / 16 / 32 sequences 46.0 / 47.8 / 47.2 us
+    // with three, 45.5 / 47.4 / 46.7 with two, 44.9 / 46.7 / 46.0 with one
     if (mode == kSkinnyNormGlu)
-        return m <= 32 ? launch_skinny_t<1, 2, 3>(ctx, w, x, m, bias, y, scratch, act, edge, mode)
+        return m <= 32 ? launch_skinny_t<1, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode)
                        : launch_skinny_t<2, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
     if (mode == kSkinnyPlain && t32 >= kWideMinTiles && (w->k == 768 || w->k == 896 || w->k == 1024)) {
         // 32 rows per launch: at m = 64 two launches, each streaming the
@@ -1684,6 +1687,9 @@ int launch_skinny(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const
     // (the fused edges never take the 4-group tiles: at t32 >= 1024 they take 2)
     if (m <= 32 || t32 < 256) {
         if (t32 >= 4 * 256 && mode == kSkinnyPlain) return launch_skinny_t<1, 4, 2>(ctx, w, x, m, bias, y, scratch, act);
+        // (the normed form on the fused SwiGLU's tile, as its bits are: 9728 x 896 at
+        // m = 32 11.9 us with three blocks per batch, 10.8 with one; 16384 x 4096 49.9 both)
+        if (t32 >= 256 && mode == kSkinnyNormIn) return launch_skinny_t<1, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
         if (t32 >= 256) return launch_skinny_t<1, 2, 3>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
         if (t32 >= 64) return launch_skinny_t<1, 1, 3>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
         return launch_skinny_t<1, 1, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
