@@ -1650,9 +1650,14 @@ constexpr size_t kWideMinTiles = 1024;
 // Tile rules from timings at m = 32 and 64 over the GPT-2 and Qwen2-0.5B
 // shapes: two column tiles per wave pay off from about 256 tiles of 32
 // columns (a 9728-wide output: 14.2 -> 11.8 us at m = 32), four only at m <=
-// 32 (four at m = 64 ran the 151936-wide head 2.8x slower); outputs narrower
-// than 2048 take one block per wave batch (more K splits, so more workgroups:
-// 896 x 896 7.9 -> 6.9 us at m = 32; a 3072-wide one slows down).  Below 256 tiles
+// 32 (four at m = 64 ran the 151936-wide head 2.8x slower).  Blocks per wave
+// batch: one for outputs narrower than 2048 (more K splits, so more workgroups:
+// 896 x 896 7.9 -> 6.9 us at m = 32) and for two column tiles (9728 x 896 at m = 32
+// 9.6 us with three, 8.9 with one; 9728 x 4096 29.9 and 25.3; with RmsNorm 9728 x 896
+// 11.9 and 10.8); between, three where the eight waves take a K of whole batches (3072
+// x 768 at m = 32: three 6.1 us, two 7.3) and two elsewhere (3072 x 1024: three
+// 8.1, two 7.1; 4096 x 4096: 18.3 and 17.4) or with the workgroups of two row
+// tiles (3072 x 768 at m = 64: three 6.2, two 5.9).  Below 256 tiles
 // of 32 columns, 33 to 64 rows are two row tiles of workgroups rather than two
 // per wave: 2304 x 768 at m = 64 10.7 -> 6.2 us, 768 x 3072 9.9 -> 8.2, a GPT-2
 // block of 64 sequences 68.2 -> 51.1; from there on one 64-row pass over the
@@ -1663,9 +1668,9 @@ int launch_skinny(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const
                   int mode = kSkinnyPlain) {
     const size_t t32 = (w->n + 31) / 32;
     // the fused SwiGLU needs each workgroup's two column groups to be a gate / up
-    // pair; one Q8_0 block per wave batch (four batches of a 896-deep K per wave) beats
-    // two and three: a Qwen2 block of 3 / 16 / 32 sequences 46.0 / 47.8 / 47.2 us
-    // with three, 45.5 / 47.4 / 46.7 with two, 44.9 / 46.7 / 46.0 with one
+    // pair; one Q8_0 block per wave batch as in the normed form, which then gives the
+    // same bits: a Qwen2 block of 3 / 16 / 32 sequences 46.0 / 47.8 / 47.2 us with
+    // three, 45.5 / 47.4 / 46.7 with two, 44.9 / 46.7 / 46.0 with one
     if (mode == kSkinnyNormGlu)
         return m <= 32 ? launch_skinny_t<1, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode)
                        : launch_skinny_t<2, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
@@ -1687,11 +1692,10 @@ int launch_skinny(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const
     // (the fused edges never take the 4-group tiles: at t32 >= 1024 they take 2)
     if (m <= 32 || t32 < 256) {
         if (t32 >= 4 * 256 && mode == kSkinnyPlain) return launch_skinny_t<1, 4, 2>(ctx, w, x, m, bias, y, scratch, act);
-        // (the normed form on the fused SwiGLU's tile, as its bits are: 9728 x 896 at
-        // m = 32 11.9 us with three blocks per batch, 10.8 with one; 16384 x 4096 49.9 both)
-        if (t32 >= 256 && mode == kSkinnyNormIn) return launch_skinny_t<1, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
-        if (t32 >= 256) return launch_skinny_t<1, 2, 3>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
-        if (t32 >= 64) return launch_skinny_t<1, 1, 3>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
+        if (t32 >= 256) return launch_skinny_t<1, 2, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
+        if (t32 >= 64 && m <= 32 && w->k % (24 * 32) == 0)
+            return launch_skinny_t<1, 1, 3>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
+        if (t32 >= 64) return launch_skinny_t<1, 1, 2>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
         return launch_skinny_t<1, 1, 1>(ctx, w, x, m, bias, y, scratch, act, edge, mode);
     }
     if (t32 >= 4 * 256 && mode == kSkinnyPlain) return launch_skinny_t<2, 2, 2>(ctx, w, x, m, bias, y, scratch, act);

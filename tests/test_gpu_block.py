@@ -462,10 +462,11 @@ def test_linear_normed_matches_oracle(fh, orc, m, n, k, rms, act):
 
 
 @pytest.mark.parametrize("m,n,k", [(33, 640, 768), (45, 2304, 768), (63, 96, 3072), (64, 8160, 128), (64, 8192, 128),
-                                   (34, 32, 32)])
+                                   (34, 32, 32), (20, 2080, 160), (32, 8224, 96), (31, 2048, 1536)])
 def test_two_row_tiles_of_workgroups(fh, orc, m, n, k):
     """33 to 64 rows of an output below 256 tiles of 32 columns (8192: one
-    64-row pass instead) are two row tiles of workgroups, the second ragged:
+    64-row pass instead) are two row tiles of workgroups, the second ragged; up
+    to 32 rows take one to three blocks of K per wave batch by width and K:
     the normed-in and the residual-out linear against the oracle, and that the second tile's rows read and write their own
     statistics."""
     import torch
