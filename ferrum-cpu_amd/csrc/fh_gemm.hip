@@ -1557,7 +1557,9 @@ int launch_skinny_t(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, con
         max_waves ? max_waves :
         MT * NT > 2 && tiles > static_cast<size_t>(ctx->num_cus) ? (16 / (MT * NT) < 8 ? 16 / (MT * NT) : 8) : 8;
     size_t splits = 1;
-    if (rows * tiles < static_cast<size_t>(ctx->num_cus) / 2) splits = (kb + kMaxWaves * BPW - 1) / (kMaxWaves * BPW);
+    // (two blocks per batch split as three do: a K of 24 blocks needs no workspace)
+    constexpr size_t kSplit = BPW == 2 ? 3 : BPW;
+    if (rows * tiles < static_cast<size_t>(ctx->num_cus) / 2) splits = (kb + kMaxWaves * kSplit - 1) / (kMaxWaves * kSplit);
     if (splits > static_cast<size_t>(kMaxSplits)) splits = kMaxSplits;
     const size_t bps = (kb + splits - 1) / splits;
     splits = (kb + bps - 1) / bps;  // no empty split

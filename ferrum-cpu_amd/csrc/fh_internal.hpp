@@ -155,8 +155,8 @@ int fh_launch_skinny_res_out(fh_ctx* ctx, const fh_q8_0* w, const float* x, size
 int fh_launch_residual_stats(fh_ctx* ctx, const float* t, const float* r, float* y, size_t rows, size_t n,
                              float* stats);
 int fh_launch_norm_from_stats(fh_ctx* ctx, const float* x, size_t rows, size_t k, const fh_edge& e, float* out);
-// act (FH_ACT_*) is applied to the outputs: in the skinny GEMM's epilogue at
-// m <= 64, else by the separate GELU kernel.
+// act (FH_ACT_*) is applied to the outputs, in the GEMMs' epilogues (after the
+// four-column-tile and vocabulary-wide forms by the separate GELU kernel).
 int fh_launch_gemm_w8a32(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m,
                          const float* bias, float* y, int act = FH_ACT_NONE);
 // The decode GEMV alone (m <= 2, W8A32, no workspace); -1 when the row is too
@@ -198,7 +198,7 @@ int fh_launch_add_layernorm(fh_ctx* ctx, const float* x, const float* y, float* 
 int fh_launch_attention_prefill(fh_ctx* ctx, const float* qkv, float* kc, float* vc, size_t d, size_t heads,
                                 size_t pos0, size_t rows, float* out);
 // The same for `seqs` sequences at once (sequence s: rows s * rows .. of qkv
-// and out, caches at kc / vc + s * seq_stride): head width 64 on the fp32
+// and out, caches at kc / vc + s * seq_stride): head widths 32 and 64 on the f16
 // matrix cores (fh_attn_prefill.hip), others one sequence at a time.
 int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, float* vc, size_t seq_stride,
                                      size_t d, size_t heads, size_t pos0, size_t rows, size_t seqs, float* out);
