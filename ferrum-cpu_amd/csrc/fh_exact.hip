@@ -12,8 +12,8 @@
 // names this contract for a packed Q8_0 forward
 // (q8_0_packed_forward_equals_expanded).
 //
-// One sequential sum per output is therefore fixed: k_linear_seq (fh_seq.hpp)
-// over the Q8_0 planes or the F32 rows.  The opt-in exact mode; FH_W8A32 is the
+// One sequential sum per output is therefore fixed: k_linear_seq and, for few
+// outputs, k_linear_seq_row (fh_seq.hpp) over the Q8_0 planes or the F32 rows.  The opt-in exact mode; FH_W8A32 is the
 // fast one.
 #include "fh_seq.hpp"
 
@@ -58,6 +58,23 @@ struct Q8Src {
             wt[(seg * 2 + v) * C + col] = fh_seq::f4{e[0], e[1], e[2], e[3]};
         }
     }
+    struct Row {
+        uint4 q;
+        uint16_t d;
+    };
+    __device__ __forceinline__ void load_row(int j, int p, int k, Row& r) const {
+        p = min(p, k - 16);
+        r.q = *reinterpret_cast<const uint4*>(qs + static_cast<size_t>(j) * k + p);
+        r.d = dsc[static_cast<size_t>(j) * (k >> 5) + (p >> 5)];
+    }
+    __device__ __forceinline__ fh_seq::f4 quad(const Row& r, int v) const {
+        const uint32_t word = v == 0 ? r.q.x : v == 1 ? r.q.y : v == 2 ? r.q.z : r.q.w;
+        const float d = fh_h2f(r.d);
+        float e[4];
+#pragma unroll
+        for (int b = 0; b < 4; b++) e[b] = d * static_cast<float>(static_cast<int8_t>((word >> (8 * b)) & 0xFFu));
+        return fh_seq::f4{e[0], e[1], e[2], e[3]};
+    }
 };
 
 struct F32Src {
@@ -86,7 +103,42 @@ struct F32Src {
         for (int v = 0; v < 2; v++)
             wt[(seg * 2 + v) * C + col] = in ? r.v[v] : fh_seq::f4{0.0f, 0.0f, 0.0f, 0.0f};
     }
+    struct Row {
+        fh_seq::f4 v[4];
+    };
+    __device__ __forceinline__ void load_row(int j, int p, int k, Row& r) const {
+        const auto* src = reinterpret_cast<const fh_seq::f4*>(rows + j * pitch + (p < k ? p : 0));
+#pragma unroll
+        for (int v = 0; v < 4; v++) r.v[v] = src[v];
+    }
+    __device__ __forceinline__ fh_seq::f4 quad(const Row& r, int v) const { return r.v[v]; }
 };
+
+// One row of x takes the decode form (k_linear_seq_row), and so do several where
+// its workgroups, one per row and 16 columns, are few per CU: they widen the
+// weights for their one row again, where k_linear_seq does so for 16 to 64.  us per
+// call, k_linear_seq against the decode form: up to two per CU, 768 x 3072 at m = 10
+// (480) 23.5 / 13.5, 4096 x 1024 at m = 2 (512) 8.8 / 7.4; up to three per CU, from
+// K = 2048 on, 768 x 3072 at m = 16 23.4 / 17.7, 1024 x 4096 at m = 12 30.5 / 22.0 (but
+// 4096 x 1024 at m = 3 8.8 / 9.0, 128 x 512 at m = 96 6.2 / 6.6).  F32 rows are four times
+// the bytes: up to one per CU, 768 x 3065 at m = 4 20.9 / 12.8 (at m = 16, three per CU,
+// 22.4 / 28.6).  A K of one k_linear_seq chunk stays there (4096 x 128 at m = 1
+// 4.1 / 4.5).
+template <class Src>
+void launch(fh_ctx* ctx, const Src& src, const fh_q8_0* w, const float* x, size_t m, const float* bias, float* y) {
+    const size_t tiles = (w->n + Src::C - 1) / Src::C, cus = static_cast<size_t>(ctx->num_cus);
+    const size_t per_cu = w->kind == FH_WEIGHT_F32 ? 1 : w->k >= 2048 ? 3 : 2;
+    // (the decode form's positions run up to a chunk past K in 32 bits)
+    const bool decode = (m == 1 || (m <= 65535 && tiles * m <= per_cu * cus)) && w->k > kChunk && w->k <= 0x7FFFF000u;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(m)),
+                           dim3(fh_seq::kThreads), 0, ctx->stream, src, x, bias, y, static_cast<int>(w->n),
+                           static_cast<int>(w->k));
+    };
+    if (!decode) fh_seq::launch(ctx, src, tiles, x, m, bias, y, w->n, w->k);
+    else if (tiles > 2 * cus && w->k < 2048) go(fh_seq::k_linear_seq_row<Src, 1>);
+    else go(fh_seq::k_linear_seq_row<Src, 2>);
+}
 
 }  // namespace
 
@@ -95,9 +147,9 @@ int fh_launch_linear_exact(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t
         return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: a dimension is above 2^31 - 1");
     if (w->n == 0 || m == 0) return FH_OK;
     if (w->kind == FH_WEIGHT_F32)
-        fh_seq::launch(ctx, F32Src{w->f32, w->pitch}, (w->n + Q8Src::C - 1) / Q8Src::C, x, m, bias, y, w->n, w->k);
+        launch(ctx, F32Src{w->f32, w->pitch}, w, x, m, bias, y);
     else
-        fh_seq::launch(ctx, Q8Src{w->qs, w->d}, (w->n + Q8Src::C - 1) / Q8Src::C, x, m, bias, y, w->n, w->k);
+        launch(ctx, Q8Src{w->qs, w->d}, w, x, m, bias, y);
     FH_HIP(ctx, hipGetLastError());
     return FH_OK;
 }

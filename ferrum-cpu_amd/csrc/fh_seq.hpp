@@ -26,8 +26,7 @@
 //
 // Measured (us per call; before: one row of x per workgroup and the products
 // through LDS for the exact linear, four rows with a byte read and a conversion
-// per product for the packed one): exact 768 x 3072 at m = 127 190.8 -> 34.0,
-// at m = 1 30.8 -> 21.2, 2304 x 768 at m = 256 320 -> 32.7; int4 2304 x 768 at
+// per product for the packed one): exact 768 x 3072 at m = 127 190.8 -> 34.0, 2304 x 768 at m = 256 320 -> 32.7; int4 2304 x 768 at
 // m = 127 38.2 -> 23.7, int8 4096 x 1024 at m = 512 247 -> 142.  At m = 512 that is
 // 81 % of the rate at which the vector units issue the multiplies and adds; at
 // 768 x 3072 and m = 127, where 1524 wave-wide chains meet 1024 SIMDs (two on
@@ -226,6 +225,121 @@ __global__ void __launch_bounds__(kThreads)
                     y[(row + r) * static_cast<long>(n) + col] = Src::kBiasFirst || !bias ? v : v + b0;
                 }
         }
+    }
+}
+
+// Few enough outputs that every workgroup has a CU's adders to itself (one row of
+// x, decode): the time is K times one step of the chain, so the summing wave
+// (wave 0) does nothing but the adds, and waves 1-3 form the rounded products of
+// the next chunk into LDS, as float4 of four consecutive p per column.  A
+// producer's job is 16 positions of one column: its four 16-byte writes land
+// beside its 15 neighbours', and the summing wave reads them the same way, both
+// free of bank conflicts.
+//
+// JOBS, the jobs per producer and chunk: with two the chunk is 384 positions (48 KB
+// of LDS, three workgroups per CU), long enough that the barrier, the first read
+// and the producers' load latency are a small part of it; one (24 KB, six per CU)
+// is for outputs that fill the chip many times over, where the neighbours cover
+// those waits.
+//
+// Measured against k_linear_seq, us per call at m = 1: 768 x 3072 21.3 -> 11.8 (one
+// job: 17.3, four: 12.5; the adds alone are 7.4), 3072 x 768 7.1 -> 4.9, 1024 x 4096
+// 27.4 -> 15.0; with one job 50257 x 768 28.5 -> 19.4 (two: 22.1), 151936 x 896
+// 79.7 -> 52.7 (66.4).
+//
+// Src, beside what k_linear_seq asks for (C = 16, no factor, bias last):
+//   Row, load_row(column, p, k, Row&)   the raw weights of positions p .. p + 15
+//   quad(Row, v)                        positions p + 4 v .. + 3 widened
+// Positions past K are loaded from inside the row and never summed.
+template <class Src, int JOBS>
+__global__ void __launch_bounds__(kThreads)
+    k_linear_seq_row(Src src, const float* __restrict__ x, const float* __restrict__ bias, float* __restrict__ y,
+                     int n, int k) {
+    constexpr int C = Src::C, kSegs = (kWaves - 1) * 4, kRowChunk = kSegs * 16 * JOBS, kRowGroups = kRowChunk / 4;
+    static_assert(C == 16 && !Src::kBiasFirst && !Src::kScaled, "the plain sum of 16 columns");
+    __shared__ f4 prod[2][kRowGroups * C];
+    const int tid = threadIdx.x, lane = tid & 63, c16 = tid & 15, tile = blockIdx.x;
+    const int chunks = (k + kRowChunk - 1) / kRowChunk;
+    const float* xr = x + static_cast<size_t>(blockIdx.y) * k;
+    // wave-uniform role (a scalar branch: every wave meets the same barriers)
+    if (__builtin_amdgcn_readfirstlane(tid >> 6) == 0) {
+        const int col = src.column(tile, c16, n);
+        const float b0 = bias && col >= 0 ? bias[col] : 0.0f;
+        float acc = 0.0f;
+        __syncthreads();  // chunk 0 is in LDS
+        for (int c = 0; c < chunks; c++) {
+            const f4* pb = prod[c & 1] + c16;
+            const int pn = min(kRowChunk, k - c * kRowChunk);
+            if (pn == kRowChunk) {
+#pragma unroll 32
+                for (int g = 0; g < kRowGroups; g++) {
+                    const f4 v = pb[g * C];
+                    acc = (((acc + v.x) + v.y) + v.z) + v.w;
+                }
+            } else {
+                const int gn = pn >> 2, rest = pn & 3;
+#pragma unroll 8
+                for (int g = 0; g < gn; g++) {
+                    const f4 v = pb[g * C];
+                    acc = (((acc + v.x) + v.y) + v.z) + v.w;
+                }
+                if (rest) {
+                    const f4 v = pb[gn * C];
+                    acc = acc + v.x;
+                    if (rest > 1) acc = acc + v.y;
+                    if (rest > 2) acc = acc + v.z;
+                }
+            }
+            __syncthreads();  // chunk c + 1 is in LDS; buffer c & 1 is free
+        }
+        if (lane < C && col >= 0) y[blockIdx.y * static_cast<size_t>(n) + col] = bias ? acc + b0 : acc;
+        return;
+    }
+    // The producers: column c16 of the tile, 16-position segments seg + kSegs * i.
+    const int seg = (tid - 64) >> 4, j = min(tile * C + c16, n - 1);
+    typename Src::Row w[2][JOBS];
+    float a[2][JOBS][16];
+    auto fetch = [&](auto S, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < JOBS; i++) {
+            const int p = c * kRowChunk + 16 * (seg + kSegs * i);
+            src.load_row(j, p, k, w[S][i]);
+            if (p + 16 <= k) {
+#pragma unroll
+                for (int e = 0; e < 16; e++) a[S][i][e] = xr[p + e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 16; e++) a[S][i][e] = xr[min(p + e, k - 1)];
+            }
+        }
+    };
+    auto produce = [&](auto S, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < JOBS; i++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const f4 q = src.quad(w[S][i], v);
+                prod[b][(4 * (seg + kSegs * i) + v) * C + c16] =
+                    f4{a[S][i][4 * v] * q.x, a[S][i][4 * v + 1] * q.y, a[S][i][4 * v + 2] * q.z,
+                       a[S][i][4 * v + 3] * q.w};
+            }
+    };
+    const std::integral_constant<int, 0> s0;
+    const std::integral_constant<int, 1> s1;
+    fetch(s0, 0);
+    if (chunks > 1) fetch(s1, 1);
+    produce(s0, 0);
+    __syncthreads();
+    // Step c: set c & 1 held chunk c (its products are in LDS), so it takes
+    // chunk c + 2; chunk c + 1's products go to buffer (c + 1) & 1.
+    auto step = [&](auto S, int c) __attribute__((always_inline)) {
+        if (c + 2 < chunks) fetch(S, c + 2);
+        if (c + 1 < chunks) produce(std::integral_constant<int, 1 - S>{}, (c + 1) & 1);
+        __syncthreads();
+    };
+    for (int c = 0; c < chunks; c += 2) {
+        step(s0, c);
+        if (c + 1 < chunks) step(s1, c + 1);
     }
 }
 

@@ -131,3 +131,31 @@ def test_exact_rows_per_lane_and_ragged_edges(fh, orc, m, n, k, f32):
     got = ferrum_hip.linear_forward(fh, x, w, b, numerics=ferrum_hip.W8A32_EXACT)
     w.free()
     bits_equal(got, want)
+
+
+# The decode form (one row, or a few workgroups per CU): K below, at and past its
+# chunks (192 positions for a wide output, 384) and 16-position jobs, an odd and an
+# even number of chunks, ragged columns, several rows, and both sides of the limit
+# of two workgroups per CU and, from K = 2048, three.
+@pytest.mark.parametrize("m,n,k", [(1, 15, 160), (1, 33, 384), (2, 16, 416), (5, 130, 768), (3, 47, 1184),
+                                   (64, 126, 160), (65, 126, 160), (96, 125, 2048), (97, 125, 2048),
+                                   (1, 8193, 192), (1, 8209, 416), (1, 8209, 608)])
+@pytest.mark.parametrize("f32", [0, 5, 15])
+def test_exact_few_outputs(fh, orc, m, n, k, f32):
+    import ferrum_hip
+
+    rng = np.random.default_rng(m + n + k + f32)
+    k -= f32
+    x = rng.standard_normal((m, k), dtype=np.float32)
+    x[m - 1, k - 1], x[m // 2, 0] = np.inf, -0.0
+    b = rng.standard_normal(n, dtype=np.float32) if m != 2 else None
+    if f32:
+        rows = (rng.standard_normal((n, k)) * 0.05).astype(np.float32)
+        rows[n - 1, k - 1] = np.nan
+        w, want = ferrum_hip.Q8_0Weight.upload_f32(fh, rows), orc.linear_forward(x, np.ascontiguousarray(rows.T), b)
+    else:
+        raw = orc.quantize_weight(n, k, m, 0.02)
+        w, want = ferrum_hip.Q8_0Weight.upload(fh, raw, n, k), reference(orc, x, raw, n, k, b)
+    got = ferrum_hip.linear_forward(fh, x, w, b, numerics=ferrum_hip.W8A32_EXACT)
+    w.free()
+    bits_equal(got, want)
