@@ -423,7 +423,10 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
 #pragma unroll
                 for (int v = 0; v < 16; v++) pw[acc_row(v, half) * 33 + col] = sv[v];
                 __builtin_amdgcn_wave_barrier();
-                for (int kk = 0; kk < kKeys && k0 + kk <= qpos; kk++) {
+                // (lanes past the block's last row have a position past its last
+                // key; they stop there, and store nothing)
+                const int last = min(qpos, kmax);
+                for (int kk = 0; kk < kKeys && k0 + kk <= last; kk++) {
                     const float p = pw[kk * 33 + col];
                     const float* vrow = key_row(k0 + kk, 2 * a.kv_dim, vc);
 #pragma unroll

@@ -821,3 +821,34 @@ def test_prompt_attention_on_every_chain_and_width(fh, orc, d, heads, seqs, rows
             want = orc.attention_decode(qkv[s * rows + r], ko, vo, heads, pos0 + r)
             close(got[s * rows + r], want, 1e-5)
         assert np.array_equal(host(fh, tk)[s], ko) and np.array_equal(host(fh, tv)[s], vo)
+
+
+# A value of v that the split products do not take (2^15 and more, inf, NaN) in
+# the last, ragged key tile of the last sequence, with and without earlier
+# positions: the lanes past the block's last row walk no key past its last one.
+# The q|k|v rows are the leading part of a larger tensor whose rest is NaN.
+@pytest.mark.parametrize("d,heads", [(128, 2), (64, 2)])
+@pytest.mark.parametrize("rows,pos0", [(1, 0), (33, 0), (129, 0), (1, 40), (33, 31), (129, 70)])
+@pytest.mark.parametrize("big", [4e4, np.inf, np.nan])
+def test_prompt_attention_large_v_in_the_last_ragged_tile(fh, orc, d, heads, rows, pos0, big):
+    import ferrum_hip
+
+    seqs, cap = 2, pos0 + rows
+    rng = np.random.default_rng(d + rows + pos0)
+    qkv = np.full((seqs * rows + 64, 3 * d), np.nan, np.float32)
+    qkv[:seqs * rows] = (rng.standard_normal((seqs * rows, 3 * d)) * 1.5).astype(np.float32)
+    kc, vc = (rng.standard_normal((seqs, cap, d)).astype(np.float32) for _ in range(2))
+    qkv[seqs * rows - 1, 2 * d + 5] = big
+    tk, tv = dev(kc), dev(vc)
+    out = dev(np.zeros((seqs * rows, d), np.float32))
+    ready()
+    ferrum_hip.attention_prefill_seqs_async(fh, dev(qkv), tk, tv, cap * d, cap, d, heads, pos0, rows, seqs, out)
+    got = host(fh, out)
+    for s in range(seqs):
+        ko, vo = kc[s].copy(), vc[s].copy()
+        for r in range(rows):
+            want = orc.attention_decode(qkv[s * rows + r], ko, vo, heads, pos0 + r)
+            fin = np.isfinite(want)
+            assert np.array_equal(np.isnan(got[s * rows + r]), np.isnan(want))
+            assert np.array_equal(got[s * rows + r][np.isinf(want)], want[np.isinf(want)])
+            close(got[s * rows + r][fin], want[fin], 1e-5)
