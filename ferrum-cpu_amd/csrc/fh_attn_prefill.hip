@@ -9,7 +9,7 @@
 // before the block come from the caches, the block's own from its q|k|v rows;
 // the same launch writes the block's k / v rows into the caches.
 //
-// How (head widths 32 and 64): one workgroup per (128 query rows, head, sequence).
+// How (head width 64): one workgroup per (128 query rows, head, sequence).
 // Each of its four waves owns 32 query rows and walks 32-key tiles of the
 // sequence's cache up to its last row's position; the tiles are staged in LDS
 // once for the four waves (double-buffered, the next tile's loads in flight
@@ -28,6 +28,7 @@ namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
+constexpr int kHd = 64;        // head width
 constexpr int kKeys = 32;      // keys per tile
 constexpr int kRT = 4;         // waves of 32 query rows that share a key tile
 constexpr int kPT = 64 * kRT, kQRows = 32 * kRT;
@@ -75,6 +76,7 @@ __device__ __forceinline__ int acc_row(int v, int half) { return (v >> 2) * 8 + 
 // instructions, shuffles through LDS for every row maximum and an LDS round trip
 // for the rescaling before).  32 prompts of 511 rows, 12 heads: 176 -> 106 us, of
 // which the order of the row groups (see the kernel) 40.
+constexpr int kHPitch = kHd + 8;    // K tile row pitch (halves): 16-byte pieces of 8 rows on different banks
 constexpr int kVPitch = kKeys + 8;  // V tile (transposed) row pitch (halves): 80-byte rows
 
 typedef _Float16 h8f __attribute__((ext_vector_type(8)));
@@ -128,35 +130,29 @@ __device__ __forceinline__ float max_halves(float v) {
     const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), false, false);
     return fmaxf(__builtin_bit_cast(float, static_cast<int>(r[0])), __builtin_bit_cast(float, static_cast<int>(r[1])));
 }
-// The largest value of each group of N = 8 or 16 lanes (xor 1, xor 2, half mirror, mirror), by
-// DPP operands.
+// The largest value of each 16-lane row (xor 1, xor 2, half mirror, mirror), by DPP operands.
 template <int CTRL>
 __device__ __forceinline__ float dpp_of(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
-template <int N>
 __device__ __forceinline__ float max_row(float v) {
     v = fmaxf(v, dpp_of<0xB1>(v));
     v = fmaxf(v, dpp_of<0x4E>(v));
     v = fmaxf(v, dpp_of<0x141>(v));
-    return N == 16 ? fmaxf(v, dpp_of<0x140>(v)) : v;
+    return fmaxf(v, dpp_of<0x140>(v));
 }
 
-// HD: the head width, 32 or 64.  HALVES = 2: eight waves, the first four on the
-// even key tiles and the others on the odd ones of the same 128 query rows, their
-// sums merged at the end (a wave's walk over its tiles is a chain: half as long,
-// where there are too few workgroups to fill the waves' waits with one another's
-// work).
-template <int HD, int HALVES>
+// HALVES = 2: eight waves, the first four on the even key tiles and the others on
+// the odd ones of the same 128 query rows, their sums merged at the end (a wave's
+// walk over its tiles is a chain: half as long, where there are too few workgroups
+// to fill the waves' waits with one another's work).
+template <int HALVES>
 __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs a) {
-    constexpr int kHPitch = HD + 8;          // K tile row pitch (halves): 16-byte pieces of 8 rows on different banks
-    constexpr int R4 = HD / 4;               // threads (float4s) per key row
-    constexpr int NK = kKeys * R4 / kPT;     // float4s of k per thread and tile
-    constexpr int KI = HD / 16, OT = HD / 32;  // MFMA K steps of a score, 32-dim output tiles
+    constexpr int KI = kHd / 16, OT = kHd / 32;  // MFMA K steps of a score, 32-dim output tiles
     // one key tile, and per wave the P of a tile with unsafe v ([key][query])
     struct Stage {
         __align__(16) _Float16 kh[2][kKeys * kHPitch], kl[2][kKeys * kHPitch];
-        __align__(16) _Float16 vh[2][HD * kVPitch], vl[2][HD * kVPitch];
+        __align__(16) _Float16 vh[2][kHd * kVPitch], vl[2][kHd * kVPitch];
         __align__(16) float kinv[2][kKeys];  // 2^-ek per key row
         __align__(16) float pt[kRT][kKeys * 33];
         int unsafe[3];                       // a tile's v is not safe for the split (step st: st % 3)
@@ -183,17 +179,17 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
     const int kmax = a.pos0 + last_row;
     const int ntiles = kmax / kKeys + 1;
     const int my_tiles = r0 < a.rows ? (a.pos0 + min(a.rows - 1, r0 + 31)) / kKeys + 1 : 0;
-    const size_t sbase = static_cast<size_t>(s) * a.seq_stride + static_cast<size_t>(h) * HD;
+    const size_t sbase = static_cast<size_t>(s) * a.seq_stride + static_cast<size_t>(h) * kHd;
     float* kc = a.kc + sbase;
     float* vc = a.vc + sbase;
 
-    // This lane's query: dims 16 i + 8 half + (0..7), i < HD / 16 (the B
+    // This lane's query: dims 16 i + 8 half + (0..7), i < 4 (the B
     // operand of step i), scaled by the row's power of two and split.
     h8f qh[KI], ql[KI];
     float qscale;
     {
         const int row = min(r0 + col, a.rows - 1);
-        const float* qp = a.qkv + (static_cast<size_t>(s) * a.rows + row) * a.ld + h * HD + half * 8;
+        const float* qp = a.qkv + (static_cast<size_t>(s) * a.rows + row) * a.ld + h * kHd + half * 8;
         float qv[8 * KI];
 #pragma unroll
         for (int i = 0; i < KI; i++) {
@@ -230,65 +226,61 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
     // also writes the block's k and v rows into the cache as it stages them
     // (no other workgroup of the launch reads those cache rows).
     const bool writer = g == a.groups - 1;
-    const float* bq = a.qkv + static_cast<size_t>(s) * a.rows * a.ld + h * HD;  // this sequence's block rows
+    const float* bq = a.qkv + static_cast<size_t>(s) * a.rows * a.ld + h * kHd;  // this sequence's block rows
     // The v rows go by pairs instead: thread t takes keys 2 (t / 16) and
-    // 2 (t / 16) + 1 (and so on kPT / 8 keys further), dims 4 (t % 16) ..., which sit side by side in the
+    // 2 (t / 16) + 1, dims 4 (t % 16) ..., which sit side by side in the
     // transposed tile, so each dim is one 4-byte store per term.
-    float4 pk[NK], pv[2];
-    const bool v_mine = HD == 64 || tid < kPT / 2;  // (wave-uniform)
+    float4 pk[2], pv[2];
     auto key_row = [&](int key, int off, const float* cache) __attribute__((always_inline)) {
         return key >= a.pos0 ? bq + static_cast<size_t>(key - a.pos0) * a.ld + off
                              : cache + static_cast<size_t>(key) * a.kv_dim;
     };
-    const int c0 = tid % R4 * 4;
-    auto k_key = [&](int i) { return tid / R4 + i * (kPT / R4); };
-    auto v_key = [&](int i) { return 2 * (tid / R4) + i; };  // (v_mine)
+    const int c0 = tid % 16 * 4;
+    auto k_key = [&](int i) { return tid / 16 + i * (kPT / 16); };
+    auto v_key = [&](int i) { return 2 * (tid / 16) + i; };
     const float* bk = bq + a.kv_dim + c0;
     const float* bv = bq + 2 * a.kv_dim + c0;
     auto fetch = [&](int t) __attribute__((always_inline)) {
         if (t * kKeys >= a.pos0) {  // (uniform) every key is the block's own
             const int r = t * kKeys - a.pos0, last = kmax - a.pos0;
 #pragma unroll
-            for (int i = 0; i < NK; i++)
+            for (int i = 0; i < 2; i++)
                 pk[i] = *reinterpret_cast<const float4*>(bk + static_cast<size_t>(min(r + k_key(i), last)) * a.ld);
-            if (v_mine)
 #pragma unroll
-                for (int i = 0; i < 2; i++)
-                    pv[i] = *reinterpret_cast<const float4*>(bv + static_cast<size_t>(min(r + v_key(i), last)) * a.ld);
+            for (int i = 0; i < 2; i++)
+                pv[i] = *reinterpret_cast<const float4*>(bv + static_cast<size_t>(min(r + v_key(i), last)) * a.ld);
             return;
         }
 #pragma unroll
-        for (int i = 0; i < NK; i++)
+        for (int i = 0; i < 2; i++)
             pk[i] = *reinterpret_cast<const float4*>(key_row(min(t * kKeys + k_key(i), kmax), a.kv_dim, kc) + c0);
-        if (v_mine)
 #pragma unroll
-            for (int i = 0; i < 2; i++)
-                pv[i] = *reinterpret_cast<const float4*>(key_row(min(t * kKeys + v_key(i), kmax), 2 * a.kv_dim, vc) + c0);
+        for (int i = 0; i < 2; i++)
+            pv[i] = *reinterpret_cast<const float4*>(key_row(min(t * kKeys + v_key(i), kmax), 2 * a.kv_dim, vc) + c0);
     };
     auto store_block_rows = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < NK; i++) {
+        for (int i = 0; i < 2; i++) {
             const int key = t * kKeys + k_key(i);
             if (key >= a.pos0 && key <= kmax)
                 *reinterpret_cast<float4*>(kc + static_cast<size_t>(key) * a.kv_dim + c0) = pk[i];
         }
-        if (v_mine)
 #pragma unroll
-            for (int i = 0; i < 2; i++) {
-                const int key = t * kKeys + v_key(i);
-                if (key >= a.pos0 && key <= kmax)
-                    *reinterpret_cast<float4*>(vc + static_cast<size_t>(key) * a.kv_dim + c0) = pv[i];
-            }
+        for (int i = 0; i < 2; i++) {
+            const int key = t * kKeys + v_key(i);
+            if (key >= a.pos0 && key <= kmax)
+                *reinterpret_cast<float4*>(vc + static_cast<size_t>(key) * a.kv_dim + c0) = pv[i];
+        }
     };
     auto stash = [&](int st) __attribute__((always_inline)) {
         const int buf = st & 1;
 #pragma unroll
-        for (int i = 0; i < NK; i++) {
+        for (int i = 0; i < 2; i++) {
             const int row = k_key(i);
             const float4 k4 = pk[i];
             // fmaxf skips NaN (whose terms are NaN without a guard, as its
             // score is); an infinite maximum takes the rare guarded path.
-            float mx = max_row<R4>(fmaxf(fmaxf(fabsf(k4.x), fabsf(k4.y)), fmaxf(fabsf(k4.z), fabsf(k4.w))));
+            float mx = max_row(fmaxf(fmaxf(fabsf(k4.x), fabsf(k4.y)), fmaxf(fabsf(k4.z), fabsf(k4.w))));
             int ek;
             h2f h01, l01, h23, l23;
             if (__builtin_expect(__ballot(!__builtin_isfinite(mx)) != 0, 0)) {
@@ -297,7 +289,7 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
                 if (__builtin_isfinite(k4.y)) fm = fmaxf(fm, fabsf(k4.y));
                 if (__builtin_isfinite(k4.z)) fm = fmaxf(fm, fabsf(k4.z));
                 if (__builtin_isfinite(k4.w)) fm = fmaxf(fm, fabsf(k4.w));
-                ek = pow2_exponent(max_row<R4>(fm));
+                ek = pow2_exponent(max_row(fm));
                 split2<true>(k4.x, k4.y, pow2f(ek), h01, l01);
                 split2<true>(k4.z, k4.w, pow2f(ek), h23, l23);
             } else {
@@ -311,7 +303,6 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
                 make_uint2(__builtin_bit_cast(uint32_t, l01), __builtin_bit_cast(uint32_t, l23));
             if (c0 == 0) kinv[buf][row] = pow2f(-ek);
         }
-        if (!v_mine) return;
         const int kp = vkey_pos(v_key(0));  // even; the pair's second key at kp + 1
         const float va[4] = {pv[0].x, pv[0].y, pv[0].z, pv[0].w};
         const float vb[4] = {pv[1].x, pv[1].y, pv[1].z, pv[1].w};
@@ -471,7 +462,7 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
     // dims 8 a + 4 half + (0..3) of both 32-dim halves of query row col
     const int row = r0 + col;
     if (row >= a.rows) return;
-    float* op = a.out + (static_cast<size_t>(s) * a.rows + row) * a.out_ld + h * HD + half * 4;
+    float* op = a.out + (static_cast<size_t>(s) * a.rows + row) * a.out_ld + h * kHd + half * 4;
 #pragma unroll
     for (int d = 0; d < OT; d++)
 #pragma unroll
@@ -487,10 +478,14 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, float* vc, size_t seq_stride,
                                      size_t d, size_t heads, size_t pos0, size_t rows, size_t seqs, float* out) {
     const size_t hd = d / heads;
-    const bool mfma = (hd == 32 || hd == 64) && aligned16(qkv) && aligned16(kc) && aligned16(vc) &&
+    const bool mfma = hd == static_cast<size_t>(kHd) && aligned16(qkv) && aligned16(kc) && aligned16(vc) &&
                       aligned16(out) && seq_stride % 4 == 0;
     if (!mfma) {
-        // other head widths: the vector-unit kernel, one sequence at a time
+        // other head widths: the vector-unit kernel, one sequence at a time.
+        // (Not width 32 either: there the two f16 terms lose bits that it keeps,
+        // 1.27e-7 of float64 against 8.8e-8 over 17 shapes, and 3.2e-6 against 8.8e-8
+        // with v a hundredth as large; and a row after 700 cached ones took 23.9 us
+        // against 8.0, its chain of tiles being one workgroup's.)
         for (size_t s = 0; s < seqs; s++) {
             const int rc = fh_launch_attention_prefill(ctx, qkv + s * rows * 3 * d, kc + s * seq_stride,
                                                        vc + s * seq_stride, d, heads, pos0, rows, out + s * rows * d);
@@ -515,7 +510,7 @@ int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, f
     a.heads = static_cast<int>(heads);
     a.pairs = static_cast<int>(pairs);
     a.groups = static_cast<int>(groups);
-    // One or two chains of key tiles per row.  Measured (ns, head width 64): a
+    // One or two chains of key tiles per row.  Measured (ns): a
     // workgroup takes 2200 per tile alone on its CU, a CU of two 1750 per tile;
     // with two chains 1500 alone (one workgroup per CU) and 2300, and 1500 for the
     // merge.  8 sequences of 300 rows and 12 heads (288 workgroups of 4, 8 and 10
@@ -530,8 +525,7 @@ int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, f
         hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(pairs * groups)), dim3(static_cast<unsigned>(kPT * halves)), 0,
                            ctx->stream, a);
     };
-    if (hd == 64) two < one ? go(k_attn_prefill_f16<64, 2>, 2) : go(k_attn_prefill_f16<64, 1>, 1);
-    else two < one ? go(k_attn_prefill_f16<32, 2>, 2) : go(k_attn_prefill_f16<32, 1>, 1);
+    two < one ? go(k_attn_prefill_f16<2>, 2) : go(k_attn_prefill_f16<1>, 1);
     FH_HIP(ctx, hipGetLastError());
     return FH_OK;
 }

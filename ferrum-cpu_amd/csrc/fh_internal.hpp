@@ -198,7 +198,7 @@ int fh_launch_add_layernorm(fh_ctx* ctx, const float* x, const float* y, float* 
 int fh_launch_attention_prefill(fh_ctx* ctx, const float* qkv, float* kc, float* vc, size_t d, size_t heads,
                                 size_t pos0, size_t rows, float* out);
 // The same for `seqs` sequences at once (sequence s: rows s * rows .. of qkv
-// and out, caches at kc / vc + s * seq_stride): head widths 32 and 64 on the f16
+// and out, caches at kc / vc + s * seq_stride): head width 64 on the f16
 // matrix cores (fh_attn_prefill.hip), others one sequence at a time.
 int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, float* vc, size_t seq_stride,
                                      size_t d, size_t heads, size_t pos0, size_t rows, size_t seqs, float* out);
