@@ -40,7 +40,7 @@ struct PrefillArgs {
     float* vc;
     size_t seq_stride;
     int kv_dim;
-    int rows, pos0, groups, heads, pairs;  // groups of kQRows query rows; pairs = heads x sequences
+    int rows, pos0;
     float scale;
     float* out;         // row s * rows + r; head h at column h * 64
     int out_ld;
@@ -172,8 +172,8 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
     // The longest rows of every head and sequence first.  (With a head's row
     // groups next to each other, a group count of four or eight gave each XCD
     // groups of one length, since workgroups are dealt to the eight in turn.)
-    const int g = a.groups - 1 - static_cast<int>(blockIdx.x) / a.pairs, pair = static_cast<int>(blockIdx.x) % a.pairs;
-    const int h = pair % a.heads, s = pair / a.heads;
+    const int groups = static_cast<int>(gridDim.z), g = groups - 1 - static_cast<int>(blockIdx.z);
+    const int h = blockIdx.x, s = blockIdx.y;
     const int r0 = g * kQRows + wave * 32;
     const int last_row = min(a.rows - 1, g * kQRows + kQRows - 1);
     const int kmax = a.pos0 + last_row;
@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
     // the cache; the last row group's workgroup of each (sequence, head), which walks every tile,
     // also writes the block's k and v rows into the cache as it stages them
     // (no other workgroup of the launch reads those cache rows).
-    const bool writer = g == a.groups - 1;
+    const bool writer = g == groups - 1;
     const float* bq = a.qkv + static_cast<size_t>(s) * a.rows * a.ld + h * kHd;  // this sequence's block rows
     // The v rows go by pairs instead: thread t takes keys 2 (t / 16) and
     // 2 (t / 16) + 1, dims 4 (t % 16) ..., which sit side by side in the
@@ -506,10 +506,6 @@ int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, f
     a.out = out;
     a.out_ld = static_cast<int>(d);
     const size_t cus = static_cast<size_t>(ctx->num_cus), pairs = heads * seqs, groups = (rows + kQRows - 1) / kQRows;
-    if (pairs * groups > 0x7FFFFFFFu) return fh_fail(ctx, FH_ERR_LIMIT, "attention_prefill: too many heads and sequences");
-    a.heads = static_cast<int>(heads);
-    a.pairs = static_cast<int>(pairs);
-    a.groups = static_cast<int>(groups);
     // One or two chains of key tiles per row.  Measured (ns): a
     // workgroup takes 2200 per tile alone on its CU, a CU of two 1750 per tile;
     // with two chains 1500 alone (one workgroup per CU) and 2300, and 1500 for the
@@ -522,8 +518,9 @@ int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, f
     const size_t one = longest * 2200 > share * 1750 ? longest * 2200 : share * 1750;
     const size_t two = (longest * 1500 > share * 2300 ? longest * 1500 : share * 2300) + 1500;
     auto go = [&](auto kern, int halves) {
-        hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(pairs * groups)), dim3(static_cast<unsigned>(kPT * halves)), 0,
-                           ctx->stream, a);
+        // (at most 65535 sequences and 512 groups of rows: the callers' limits)
+        hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(heads), static_cast<unsigned>(seqs), static_cast<unsigned>(groups)),
+                           dim3(static_cast<unsigned>(kPT * halves)), 0, ctx->stream, a);
     };
     two < one ? go(k_attn_prefill_f16<2>, 2) : go(k_attn_prefill_f16<1>, 1);
     FH_HIP(ctx, hipGetLastError());

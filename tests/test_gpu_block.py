@@ -874,3 +874,26 @@ def test_prompt_attention_of_small_v_at_width_32(fh):
     e = np.exp(s - s.max(axis=-1, keepdims=True))
     want = (e / e.sum(axis=-1, keepdims=True) @ v).transpose(0, 2, 1, 3)
     assert np.abs(got - want).max() <= 1e-6 * np.abs(want).max()
+
+
+def test_prompt_attention_of_more_workgroups_than_one_grid_dimension_holds(fh):
+    """65535 sequences of 257 heads: 2^24 and more workgroups, whose threads no
+    single grid dimension can count.  One position each, so every output is its
+    v row (two f16 terms of it: 2^-22 of values below 8)."""
+    import torch
+
+    import ferrum_hip
+
+    seqs, heads = 65535, 257
+    d = 64 * heads
+    qkv = torch.zeros((seqs, 3 * d), device="cuda")
+    qkv[:, 2 * d:] = torch.rand((seqs, d), device="cuda") * 8 - 4
+    kc, vc, out = (torch.full((seqs, d), float("nan"), device="cuda") for _ in range(3))
+    ready()
+    ferrum_hip.attention_prefill_seqs_async(fh, qkv, kc, vc, d, 1, d, heads, 0, 1, seqs, out)
+    fh.sync()
+    assert torch.equal(vc, qkv[:, 2 * d:])
+    assert (out - vc).abs().max().item() <= 8 * 2.0 ** -22
+    assert torch.equal(kc, torch.zeros_like(kc))
+    del qkv, kc, vc, out
+    torch.cuda.empty_cache()
