@@ -1,0 +1,77 @@
+"""Calls under graph capture on a context that has not run them before: what
+needs no workspace, or no more than an earlier call of the context left, can be
+captured without a run of its own, and each replay gives the eager result."""
+import contextlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@contextlib.contextmanager
+def fresh_context():
+    import ferrum_hip
+
+    ctx = ferrum_hip.Context(0)
+    try:
+        yield ctx
+    finally:
+        ctx.sync()
+        ctx.close()
+
+
+def replays_equal_eager(ctx, call, out):
+    """Capture `call` (which fills `out`) before it has run on `ctx`; three
+    replays with eager runs between them, every result the same bits."""
+    import torch
+
+    g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    try:
+        with torch.cuda.graph(g, stream=s):
+            ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+            call()
+    finally:
+        ctx.set_stream(None)
+    seen = []
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        seen.append(out.cpu().numpy().view(np.uint32).copy())
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        call()
+        ctx.sync()
+        seen.append(out.cpu().numpy().view(np.uint32).copy())
+    assert np.isfinite(seen[0].view(np.float32)).all()
+    assert all(np.array_equal(v, seen[0]) for v in seen)
+
+
+def on_device(*arrays):
+    import torch
+
+    return [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in arrays]
+
+
+# SwiGLU of a narrow model: up to 24 blocks of K it splits no K, and needs no
+# workspace.
+@pytest.mark.parametrize("m,ffn,k", [(3, 2048, 768), (32, 2048, 768), (17, 512, 288), (32, 3072, 768)])
+def test_swiglu_up_to_24_blocks_needs_no_workspace(orc, m, ffn, k):
+    import torch
+
+    import ferrum_hip
+
+    rng = np.random.default_rng(m + ffn)
+    with fresh_context() as ctx:
+        w = ferrum_hip.Q8_0Weight.upload(ctx, orc.quantize_weight(2 * ffn, k, ffn, 0.05), 2 * ffn, k)
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        grp = x.reshape(m, k // 32, 32)
+        stats = np.stack([grp.mean(2), ((grp - grp.mean(2, keepdims=True)) ** 2).sum(2)], axis=2).astype(np.float32)
+        dx, st, gam = on_device(x, stats, rng.standard_normal(k).astype(np.float32))
+        y = torch.empty((m, ffn), device="cuda")
+        replays_equal_eager(ctx, lambda: ferrum_hip.linear_normed_async(
+            ctx, w, dx, m, k, st, gam, None, 1e-6, True, None, 0, y, ferrum_hip.ACT_SWIGLU32), y)
+        w.free()
