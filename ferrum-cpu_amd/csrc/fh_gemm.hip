@@ -941,12 +941,14 @@ __global__ void __launch_bounds__(512)
     k_gemm_skinny(const float* __restrict__ x, const int8_t* __restrict__ qs, const uint16_t* __restrict__ dsc,
                   const int8_t* __restrict__ rexp, const float* __restrict__ bias, float* y, int m, int n,
                   int k, int bps, float* __restrict__ part, unsigned* __restrict__ counters, int act, fh_edge e) {
-    {  // grid.z: tiles of 32 MT rows
+    // grid.z: tiles of 32 MT rows (the fused edges' launches of 64 rows per workgroup
+    // and SwiGLU's have one)
+    if constexpr (MODE == kSkinnyPlain || (MT == 1 && MODE != kSkinnyNormGlu)) {
         const size_t rows = static_cast<size_t>(blockIdx.z) * (32 * MT);
         x += rows * k;
-        y += rows * (MODE == kSkinnyNormGlu ? n >> 1 : n);
+        y += rows * n;
         m -= static_cast<int>(rows);
-        if constexpr (MODE == kSkinnyNormIn || MODE == kSkinnyNormGlu) e.stats += rows * (k >> 5) * 2;
+        if constexpr (MODE == kSkinnyNormIn) e.stats += rows * (k >> 5) * 2;
         if constexpr (MODE == kSkinnyResOut) {
             e.r += rows * n;
             e.stats += rows * (n >> 5) * 2;
@@ -1601,6 +1603,8 @@ int launch_skinny_t(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, con
         }
     }
     if (tiles > 0x7FFFFFFFu) return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: too many output columns");
+    if (rows > 1 && mode != kSkinnyPlain && (MT > 1 || mode == kSkinnyNormGlu))
+        return fh_fail(ctx, FH_ERR_LIMIT, "skinny GEMM: one row tile with this fused edge");
     const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(splits), static_cast<unsigned>(rows)), block(static_cast<unsigned>(64 * kw));
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, block, lds, ctx->stream, x, w->qs, w->d, w->rexp, bias, y, static_cast<int>(m),
