@@ -1786,6 +1786,29 @@ int fh_launch_skinny_scratch(fh_ctx* ctx, const fh_q8_0* w, const float* x, size
     return launch_skinny(ctx, w, x, m, bias, y, &scratch);
 }
 
+// What any call of 65 to m rows over k inputs may ask of the workspace: the split
+// panel of m rows, or the K splits' partials (8 splits of one 32 x 32 tile per two
+// CUs).  Which kernel a call takes is not monotone in m (768 x 3072: K splits up to
+// 160 rows, no workspace up to 5504, then a panel), so each call makes room for all
+// the shorter ones: a program that has run its longest prompt can capture any
+// shorter one.  (Not while capturing itself; and without the memory this call
+// may still run.)
+static void reserve_shorter_prompts(fh_ctx* ctx, size_t m, size_t k) {
+    const size_t m_pad = (m + 127) / 128 * 128;
+    const size_t panel = fh_align256(m_pad * k * 4) + fh_align256(m_pad * 4) + fh_align256(m_pad);
+    const size_t partials = static_cast<size_t>(ctx->num_cus) / 2 * kMaxSplits * 1024 * sizeof(float);
+    const size_t bytes = panel > partials ? panel : partials;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (ctx->ws_bytes >= bytes || hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess ||
+        cs != hipStreamCaptureStatusNone)
+        return;
+    void* ws = nullptr;
+    if (fh_workspace(ctx, bytes, &ws) != FH_OK) {
+        (void)hipGetLastError();
+        ctx->err.clear();
+    }
+}
+
 // m <= 64 takes the skinny kernel.  Larger m takes the kernel and tile with the
 // least estimated time.  Fitted to timings over the GPT-2 and Qwen2-0.5B shapes
 // at m = 65 .. 16352 (256 CUs), with kb blocks of K:
@@ -1810,6 +1833,7 @@ int fh_launch_gemm_w8a32(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m
     const size_t t32 = tiles(32), ns32 = 4000 + kb * t32 * 42 / 100, ns64 = 5000 + kb * 620 * rounds(tiles(64), 2 * cus);
     const size_t ns128 = 5000 + kb * 1730 * rounds(tiles(128), 2 * cus);
     const size_t ns256 = 8000 + kb * 2500 * rounds(tiles(256), cus);
+    reserve_shorter_prompts(ctx, m, w->k);
     const size_t rows = (m + 31) / 32;  // (grid.z)
     const size_t skinny = t32 <= 2 * cus ? 0 : ns32 < ns64 ? ns32 : ns64, big = ns128 < ns256 ? ns128 : ns256;
     if (skinny <= big && rows <= 65535) {

@@ -75,3 +75,29 @@ def test_swiglu_up_to_24_blocks_needs_no_workspace(orc, m, ffn, k):
         replays_equal_eager(ctx, lambda: ferrum_hip.linear_normed_async(
             ctx, w, dx, m, k, st, gam, None, 1e-6, True, None, 0, y, ferrum_hip.ACT_SWIGLU32), y)
         w.free()
+
+
+# After one call at the longest prompt, any shorter one over as many inputs can be
+# captured, whichever kernel each takes: K splits (768 x 3072 at 97 rows) after
+# a call that asks for no workspace (511 rows) or for fewer partials (127), the
+# 128 x 128 tiles' panel (4096 x 1024 at 1050 rows, 50257 x 64 at 65) after
+# smaller needs.
+@pytest.mark.parametrize("n,k,longest,m", [(768, 3072, 511, 97), (1344, 3072, 127, 96), (4096, 1024, 2100, 1050),
+                                           (50257, 64, 300, 65), (768, 3072, 511, 511), (130, 96, 200, 70)])
+def test_shorter_prompts_after_the_longest(orc, n, k, longest, m):
+    import torch
+
+    import ferrum_hip
+
+    rng = np.random.default_rng(n + m)
+    with fresh_context() as ctx:
+        w = ferrum_hip.Q8_0Weight.upload(ctx, orc.quantize_weight(n, k, m, 0.05), n, k)
+        x, b = on_device(rng.standard_normal((longest, k)).astype(np.float32),
+                         rng.standard_normal(n).astype(np.float32))
+        y = torch.empty((longest, n), device="cuda")
+        torch.cuda.synchronize()
+        ferrum_hip.linear_forward_async(ctx, w, x, longest, k, b, n, y)
+        ctx.sync()
+        out = torch.empty((m, n), device="cuda")
+        replays_equal_eager(ctx, lambda: ferrum_hip.linear_forward_async(ctx, w, x, m, k, b, n, out), out)
+        w.free()
