@@ -14,10 +14,10 @@
 //
 // Device layout: the reference's row-major bytes, each row padded to a
 // multiple of 64 bytes.  Several rows of x (a prompt) run on k_linear_seq
-// (fh_seq.hpp).  With one row (k_qlinear_row, the decode case) one wave sums
-// and three form the products.  The sums are dependency chains of K adds, so
-// the columns (and rows of x) are the parallelism and the chunk pipeline keeps
-// the loads in flight meanwhile.
+// (fh_seq.hpp), a few rows of a wide output on k_qlinear.  With one row
+// (k_qlinear_row, the decode case) one wave sums and three form the products.
+// The sums are dependency chains of K adds, so the columns (and rows of x) are
+// the parallelism and the chunk pipeline keeps the loads in flight meanwhile.
 #include <type_traits>
 
 #include "fh_seq.hpp"
@@ -38,7 +38,9 @@ namespace {
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int kTile = 64;  // the rows' padding, in bytes
+constexpr int kTile = 64;    // column bytes per workgroup of k_qlinear, and the rows' padding
+constexpr int kChunk = 512;  // positions per LDS chunk of k_qlinear
+constexpr int kSegs = kChunk * kTile / 16 / kThreads;  // 16-byte row segments per thread and chunk
 
 // quant.rs:222-225 nibble_to_i8: sign-extend a 4-bit level
 __device__ __forceinline__ float level4(uint32_t b, bool hi) {
@@ -96,6 +98,96 @@ struct LevelSrc {
             }
     }
 };
+
+// A few rows of x of a wide output (launch() below): a workgroup owns one 64-byte
+// column tile of every row (64 int8 columns, or 64 low- and 64 high-nibble int4
+// columns) and M rows of x (grid.y over row groups).  It walks K in chunks of 512
+// positions: all 256 threads stream a chunk (32 KB, row segments of 16 bytes) and
+// its scaled activations into one LDS buffer while wave i sums the previous chunk
+// for x row i, one lane per column.  Against k_linear_seq it reads each level byte
+// from LDS instead of a widened float, so its step costs more (13 ns a position
+// and 64 columns of int8, 23 of int4), but it has 64 or 128 columns per workgroup
+// and every wave of M = 4 rows sums, where k_linear_seq has 16 or 32 and a tile
+// of 16 or 8 rows.  KIND 0: int8, 1: int4.
+template <int KIND, int M>
+__global__ void __launch_bounds__(kThreads)
+    k_qlinear(const uint8_t* __restrict__ q, const float* __restrict__ scales, const float* __restrict__ x,
+              const float* __restrict__ bias, float* __restrict__ y, int m, int k, int n, int pitch) {
+    static_assert(M <= kThreads / 64, "one summing wave per row");
+    __shared__ __align__(16) uint8_t wt[2][kChunk][kTile];
+    __shared__ float a[2][M][kChunk];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int c0 = blockIdx.x * kTile, row0 = blockIdx.y * M;
+    const int half = (n + 1) / 2;
+    // the column(s) lane `lane` of a summing wave owns
+    const int col_lo = c0 + lane, col_hi = half + c0 + lane;
+    const bool live_lo = KIND == 0 ? col_lo < n : col_lo < half;
+    const bool live_hi = KIND == 1 && col_hi < n;
+    const bool summing = wave < M && row0 + wave < m;
+    // every output starts at its bias (the reference fuses the bias first)
+    float acc_lo = bias && live_lo ? bias[col_lo] : 0.0f;
+    float acc_hi = bias && live_hi ? bias[col_hi] : 0.0f;
+    const int chunks = (k + kChunk - 1) / kChunk;
+    constexpr int kAPer = kChunk / kThreads;  // activation rows per thread and chunk
+    u4 seg[kSegs];
+    float xv[M][kAPer], sv[kAPer];
+    // Chunk c: thread t loads segment t % 4 of rows t / 4 + 64 j, and x and the
+    // scale of rows t + 256 j (all clamped to valid rows: rows past K are
+    // loaded, never summed).
+    auto fetch = [&](int c) __attribute__((always_inline)) {
+        const int p0 = c * kChunk;
+#pragma unroll
+        for (int j = 0; j < kSegs; j++) {
+            const int p = min(p0 + (tid >> 2) + j * (kThreads / 4), k - 1);
+            seg[j] = *reinterpret_cast<const u4*>(q + static_cast<size_t>(p) * pitch + c0 + (tid & 3) * 16);
+        }
+#pragma unroll
+        for (int j = 0; j < kAPer; j++) {
+            const int p = min(p0 + tid + j * kThreads, k - 1);
+            sv[j] = scales[p];
+#pragma unroll
+            for (int i = 0; i < M; i++) xv[i][j] = x[static_cast<size_t>(min(row0 + i, m - 1)) * k + p];
+        }
+    };
+    // a'[i, p] = x[i, p] * scale[p] (ops.rs:331-339) and the levels, into buffer b
+    auto store = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < kSegs; j++)
+            *reinterpret_cast<u4*>(&wt[b][(tid >> 2) + j * (kThreads / 4)][(tid & 3) * 16]) = seg[j];
+#pragma unroll
+        for (int j = 0; j < kAPer; j++)
+#pragma unroll
+            for (int i = 0; i < M; i++) a[b][i][tid + j * kThreads] = xv[i][j] * sv[j];
+    };
+    fetch(0);
+    store(0);
+    __syncthreads();
+    for (int c = 0; c < chunks; c++) {
+        const int b = c & 1;
+        if (c + 1 < chunks) fetch(c + 1);  // next chunk in flight during the sums
+        if (summing) {
+            const int pn = min(kChunk, k - c * kChunk);
+            const float* ar = a[b][wave];
+            for (int u = 0; u < pn; u++) {
+                const uint32_t wb = wt[b][u][lane];
+                const float ap = ar[u];
+                if (KIND == 0) {
+                    acc_lo = acc_lo + ap * static_cast<float>(static_cast<int8_t>(wb));
+                } else {
+                    acc_lo = acc_lo + ap * level4(wb, false);
+                    acc_hi = acc_hi + ap * level4(wb, true);
+                }
+            }
+        }
+        if (c + 1 < chunks) store(b ^ 1);  // the other buffer: last read two chunks ago
+        __syncthreads();
+    }
+    if (summing) {
+        float* yr = y + static_cast<size_t>(row0 + wave) * n;
+        if (live_lo) yr[col_lo] = acc_lo;
+        if (live_hi) yr[col_hi] = acc_hi;
+    }
+}
 
 // One row of x (the decode case).  A sum is a chain of K dependent adds, so
 // the time of the kernel is K times the cost of one step of that chain.  Here
@@ -262,6 +354,42 @@ __global__ void __launch_bounds__(kThreads)
     }
 }
 
+// Several rows of x: the kernel with the least estimated time, in ns.  The chains of
+// a position take the time of the CU with the most workgroups, which hold each other
+// up in the pattern below (two k_qlinear and three k_linear_seq workgroups share a
+// CU; their summing waves start on successive SIMDs).  Fitted to both kernels at n =
+// 2304 .. 151936, k = 128 .. 4096, m = 2 .. 20 and 256 CUs, 2618 calls: all but 56
+// take the faster kernel or lose under 3 % by it.  us, k_linear_seq and k_qlinear:
+// int8 16384 x 768 at m = 4 17.1 / 13.0 and at m = 16 23.3 / 30.1, int8 28672 x 512
+// at m = 2 18.2 / 9.5, int4 50257 x 768 at m = 4 28.4 / 26.4 and at m = 5 32.0 / 44.3.
+bool few_rows(int kind, size_t cus, size_t pitch, size_t row_bytes, size_t k, size_t m, size_t cols) {
+    const bool int8 = kind == FH_QINT8;
+    if (m > 64) return false;
+    const double wgs = static_cast<double>(pitch / kTile * ((m + 3) / 4)) / static_cast<double>(cus);
+    const double pairs = ceil(wgs / 2) - 1, rest = wgs - 2 * pairs;
+    const bool crowded = int8 && pairs > 0 && k > kChunk;  // (chunks of several workgroups stream at once)
+    const double last = int8 ? (rest <= 1 ? (crowded ? 14.7 : 12.7) + 1.9 * rest : crowded ? 21.0 + rest : 9.0 + 4.0 * rest)
+                             : (rest <= 1 ? 22.0 + 2.3 * rest : 21.1 + 3.9 * rest);
+    const double step = (int8 ? 16.5 : 25.5) * pairs + last;
+    const size_t bytes = int8 ? cols : cols / 2, tiles = (row_bytes + bytes - 1) / bytes;
+    const size_t tm = fh_seq::rows_per_lane(cus, cols, tiles, m);
+    const size_t rows = 64 / cols * tm, live = (m + rows - 1) / rows;  // summing waves of the first row tile
+    const size_t c = (tiles * fh_seq::row_tiles(cols, m, tm) + cus - 1) / cus;
+    const double d = static_cast<double>(c);
+    double seq;
+    if (tm > 1) seq = ((cols == 16 ? 8.5 : 9.0) * d + 3.0) * static_cast<double>(tm) / 2;
+    else if (cols == 16)
+        seq = live == 1   ? 8.3 * static_cast<double>((c + 2) / 3)
+              : live == 2 ? 12.0 * static_cast<double>(c / 3) + 5.7 * static_cast<double>(c % 3) + (c == 1 ? 2.0 : 0.0)
+                          : 4.35 * d + 3.6;
+    else
+        seq = live == 1   ? 3.2 * d + (int8 ? 5.6 : 2.0)
+              : live == 2 ? (int8 ? 4.8 * d + 2.5 : 4.0 * d + 3.0)
+                          : (int8 ? 5.2 : 4.6) * d + 4.0;
+    const double kd = static_cast<double>(k);
+    return kd * step + 1850 + 360 * wgs < kd * seq + 2500 + 283 * d;
+}
+
 template <int KIND>
 int launch(fh_ctx* ctx, const fh_qweight* w, const float* x, size_t m, const float* bias, float* y) {
     const unsigned gx = static_cast<unsigned>(w->pitch / kTile);
@@ -278,14 +406,18 @@ int launch(fh_ctx* ctx, const fh_qweight* w, const float* x, size_t m, const flo
         else
             hipLaunchKernelGGL((k_qlinear_row<KIND, 64>), dim3(gx), dim3(kThreads), 0, ctx->stream, w->q, w->scales,
                                x, bias, y, ki, ni, pi);
+    } else if (few_rows(KIND == 0 ? FH_QINT8 : FH_QINT4, static_cast<size_t>(ctx->num_cus), w->pitch, w->row_bytes, w->k, m,
+                        w->n >= 32768 ? 32 : 16)) {
+        hipLaunchKernelGGL((k_qlinear<KIND, 4>), dim3(gx, static_cast<unsigned>((m + 3) / 4)), dim3(kThreads), 0,
+                           ctx->stream, w->q, w->scales, x, bias, y, static_cast<int>(m), ki, ni, pi);
     } else {
         auto go = [&](auto src) {
             using Src = decltype(src);
             fh_seq::launch(ctx, src, (w->row_bytes + Src::kBytes - 1) / Src::kBytes, x, m, bias, y, w->n, w->k);
         };
         // 32 columns per workgroup for vocabulary heads (longer pieces of each
-        // row: int4 50257 x 768 at m = 4 27.9 against 38.7 us), 16 for layers
-        // (more workgroups: 768 x 768 8.3 against 9.0)
+        // row: int4 50257 x 768 at m = 4 27.9 us, with 16 38.7), 16 for layers
+        // (more workgroups: 768 x 768 8.3 us, with 32 9.0)
         const int half = static_cast<int>((w->n + 1) / 2);
         if (w->n >= 32768) go(LevelSrc<KIND, 32>{w->q, w->scales, pi, half});
         else go(LevelSrc<KIND, 16>{w->q, w->scales, pi, half});

@@ -349,24 +349,29 @@ __global__ void __launch_bounds__(kThreads)
 // waits: int4 4096 x 1024 at m = 127 runs 45.3 / 43.1 / 39.4 us with TM = 1 / 2 /
 // 4 (8, 4 and 2 whole rounds), 768 x 3072 41.8 / 41.7 / 67.7 (384, 192 and 96
 // workgroups).
+inline size_t row_tiles(size_t cols, size_t m, size_t tm) { return (m + kThreads / cols * tm - 1) / (kThreads / cols * tm); }
+inline size_t rows_per_lane(size_t cus, size_t cols, size_t tiles, size_t m) {
+    auto blocks = [&](size_t tm) { return tiles * row_tiles(cols, m, tm); };
+    auto cost = [&](size_t tm) { return ((blocks(tm) + cus - 1) / cus) * (20 * tm + 3); };
+    size_t tm = 1;
+    for (size_t t = 2; t <= 4; t *= 2)
+        if (blocks(t) >= 2 * cus && cost(t) < cost(tm)) tm = t;
+    return tm;
+}
+
 template <class Src>
 void launch(fh_ctx* ctx, const Src& src, size_t tiles, const float* x, size_t m, const float* bias, float* y, size_t n,
             size_t k) {
-    const size_t rows = kThreads / Src::C, cus = static_cast<size_t>(ctx->num_cus);
-    auto blocks = [&](size_t tm) { return tiles * ((m + rows * tm - 1) / (rows * tm)); };
-    auto cost = [&](size_t tm) { return ((blocks(tm) + cus - 1) / cus) * (20 * tm + 3); };
-    auto go = [&](auto kernel, size_t tm) {
-        const size_t gy = (m + rows * tm - 1) / (rows * tm);
+    const size_t tm = rows_per_lane(static_cast<size_t>(ctx->num_cus), Src::C, tiles, m);
+    auto go = [&](auto kernel) {
+        const size_t gy = row_tiles(Src::C, m, tm);
         hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((tiles + 7) / 8 * 8), static_cast<unsigned>(gy < 65535 ? gy : 65535)),
                            dim3(kThreads), 0, ctx->stream, src, x, bias, y, static_cast<int>(m), static_cast<int>(n),
                            static_cast<int>(k), static_cast<int>(tiles));
     };
-    size_t tm = 1;
-    for (size_t t = 2; t <= 4; t *= 2)
-        if (blocks(t) >= 2 * cus && cost(t) < cost(tm)) tm = t;
-    if (tm == 4) go(k_linear_seq<Src, 4>, 4);
-    else if (tm == 2) go(k_linear_seq<Src, 2>, 2);
-    else go(k_linear_seq<Src, 1>, 1);
+    if (tm == 4) go(k_linear_seq<Src, 4>);
+    else if (tm == 2) go(k_linear_seq<Src, 2>);
+    else go(k_linear_seq<Src, 1>);
 }
 
 }  // namespace fh_seq

@@ -101,3 +101,15 @@ def test_qlinear_rows_per_lane_and_ragged_edges(fh, orc, kind, m, k, n):
     w.free()
     nan = np.isnan(got) & np.isnan(want)
     assert np.array_equal(np.where(nan, 0, got.view(np.uint32)), np.where(nan, 0, want.view(np.uint32)))
+
+
+# A few rows of a wide output (k_qlinear: 64-byte column tiles, four rows of x per
+# workgroup, K in chunks of 512 positions), where the launch rule takes it over the
+# kernel above by half of its time or more: the last tile's columns ragged (odd int4
+# widths), one, three and four rows of the last group, K of one chunk, of whole chunks
+# and ending inside one, non-finite values and a sum of -0.
+@pytest.mark.parametrize("kind,m,k,n", [(0, 2, 255, 28673), (0, 3, 512, 28671), (0, 4, 130, 31999), (0, 5, 256, 16385),
+                                        (0, 8, 513, 14337), (1, 2, 129, 32001), (1, 3, 100, 28673), (1, 4, 250, 28671),
+                                        (1, 7, 129, 32001), (1, 8, 1025, 32767), (0, 4, 1537, 16384)])
+def test_qlinear_few_rows_of_a_wide_output(fh, orc, kind, m, k, n):
+    test_qlinear_rows_per_lane_and_ragged_edges(fh, orc, kind, m, k, n)
