@@ -54,6 +54,18 @@ static int grow_area(fh_ctx* ctx, void** area, size_t* area_bytes, size_t bytes,
 
 int fh_workspace(fh_ctx* ctx, size_t bytes, void** out) { return grow_area(ctx, &ctx->ws, &ctx->ws_bytes, bytes, out); }
 
+void fh_reserve_workspace(fh_ctx* ctx, size_t bytes) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (ctx->ws_bytes >= bytes || hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess ||
+        cs != hipStreamCaptureStatusNone)
+        return;
+    void* ws = nullptr;
+    if (fh_workspace(ctx, bytes, &ws) != FH_OK) {
+        (void)hipGetLastError();  // (the call that comes next asks for what it needs)
+        ctx->err.clear();
+    }
+}
+
 int fh_act_area(fh_ctx* ctx, size_t bytes, void** out) { return grow_area(ctx, &ctx->act, &ctx->act_bytes, bytes, out); }
 
 // Pinned host staging of the blocking calls (grown with hipHostMalloc; only

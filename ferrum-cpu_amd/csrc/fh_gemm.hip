@@ -693,8 +693,9 @@ __global__ void __launch_bounds__(256, 2)
     }
 }
 
-// W8A8 where 256 x 256 tiles fill the chip, the same arithmetic as k_gemm_w8a8
-// (every output the same bits): a workgroup owns a 256 x 256 output tile (eight
+// W8A8 where 256 x 256 tiles nearly fill whole rounds of the chip (and K is long, in
+// the exact mode), the same arithmetic as k_gemm_w8a8 (every output the same
+// bits): a workgroup owns a 256 x 256 output tile (eight
 // waves of 128 x 64, 4 x 2 32 x 32 tiles) and stages one Q8_0 block of it at a
 // time.  The block terms are formed on the matrix cores, leaving two VALU
 // operations per output and block, the product and the sum (FAST: one):
@@ -1716,22 +1717,32 @@ template <bool V4>
 __global__ void fh_k_encode_panel(const float* __restrict__ x, int m, int m_pad, int kb, uint4* __restrict__ qp,
                                   float* __restrict__ dp);
 
+// ns of k_gemm_w8a8, encode included: a chain of kb blocks in each workgroup (and
+// fewer rows to encode below 30), or the whole chip's outputs, with a tile's start
+// and end.  Beside it, the 256 x 256 tiles take 7 us and 16.3 us + 1.88 us per
+// block (fast mode: 15.3, 1.52) per round of one workgroup per CU.  Fitted at 256 CUs
+// to n = 128 .. 151936, k = 96 .. 4864, m = 4 .. 16384 in both modes: of 296 calls
+// where both tiles come into question none takes one 4 % slower than the other.  us, 64 x 64 tiles and 256 x
+// 256 ones: 4096 x 1024 at m = 4079 81.3 / 82.7, fast 76.1 / 70.9; 4096 x 4096 at m =
+// 8175 550 / 521, fast 508 / 436; 2304 x 768 at m = 7151 67.0 / 70.5.
+size_t fh_w8a8_tile_ns(size_t m, size_t n, size_t kb, bool fast) {
+    const size_t t32 = (m + 31) / 32 * ((n + 31) / 32);
+    const size_t chain = 5700 + 40 * (m < 30 ? m : 30) + (fast ? 220 : 240) * kb;
+    const size_t chip = fast ? 4500 + t32 * (114 * kb + 750) / 1000 : 6500 + t32 * (122 * kb + 730) / 1000;
+    return chain > chip ? chain : chip;
+}
+
 // W8A8 through the int8 matrix cores: the activations are encoded into the
 // lane-order panel, then the GEMM.
 int fh_launch_gemm_w8a8(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const float* bias, float* y,
                         bool fast) {
-    // Two kernels, the one with the least time.  Measured (ns per block of K, 256
-    // CUs): the 64 x 64 workgroup tile 250 + 0.13 per 32 x 32 of output; the 256 x
-    // 256 one 2300 per round of one workgroup per CU, 2100 in the fast mode.  4096
-    // x 1024 at m = 4096 (one round): 80.4 us and 82.1, fast 77.0 and 69.2; 1024 x
-    // 4096 at m = 16352 (one round): 322.9 and 307.2; 768 x 3072 at m = 2048 (24
-    // tiles of 256 x 256 for the 256 CUs): 39.9 and 190.
-    const size_t cus = static_cast<size_t>(ctx->num_cus);
-    const size_t t32 = (m + 31) / 32 * ((w->n + 31) / 32);
-    const size_t t256 = (m + kW8Rows - 1) / kW8Rows * ((w->n + kW8Cols - 1) / kW8Cols);
-    const bool staged = (t256 + cus - 1) / cus * (fast ? 2100 : 2300) < 250 + t32 * 130 / 1000;
+    // (64 x 64 tiles or 256 x 256 ones, whichever should take less: fh_w8a8_tile_ns)
+    const size_t kb = w->k / 32;
+    const size_t rounds = ((m + kW8Rows - 1) / kW8Rows * ((w->n + kW8Cols - 1) / kW8Cols) + ctx->num_cus - 1) / ctx->num_cus;
+    const bool staged = 7000 + rounds * (fast ? 1520 * kb + 15300 : 1880 * kb + 16300) < fh_w8a8_tile_ns(m, w->n, kb, fast);
     const int tm_rows = staged ? kW8Rows : 64;
-    const size_t kb = w->k / 32, m_pad = (m + tm_rows - 1) / tm_rows * tm_rows;
+    fh_reserve_workspace(ctx, fh_w8a8_workspace(m, w->k));
+    const size_t m_pad = (m + tm_rows - 1) / tm_rows * tm_rows;
     const size_t qbytes = fh_align256(m_pad * w->k), dbytes = fh_align256(m_pad * kb * 4);
     void* ws = nullptr;
     int rc = fh_workspace(ctx, qbytes + dbytes, &ws);
@@ -1791,22 +1802,12 @@ int fh_launch_skinny_scratch(fh_ctx* ctx, const fh_q8_0* w, const float* x, size
 // CUs).  Which kernel a call takes is not monotone in m (768 x 3072: K splits up to
 // 160 rows, no workspace up to 5504, then a panel), so each call makes room for all
 // the shorter ones: a program that has run its longest prompt can capture any
-// shorter one.  (Not while capturing itself; and without the memory this call
-// may still run.)
+// shorter one.
 static void reserve_shorter_prompts(fh_ctx* ctx, size_t m, size_t k) {
     const size_t m_pad = (m + 127) / 128 * 128;
     const size_t panel = fh_align256(m_pad * k * 4) + fh_align256(m_pad * 4) + fh_align256(m_pad);
     const size_t partials = static_cast<size_t>(ctx->num_cus) / 2 * kMaxSplits * 1024 * sizeof(float);
-    const size_t bytes = panel > partials ? panel : partials;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (ctx->ws_bytes >= bytes || hipStreamIsCapturing(ctx->stream, &cs) != hipSuccess ||
-        cs != hipStreamCaptureStatusNone)
-        return;
-    void* ws = nullptr;
-    if (fh_workspace(ctx, bytes, &ws) != FH_OK) {
-        (void)hipGetLastError();
-        ctx->err.clear();
-    }
+    fh_reserve_workspace(ctx, panel > partials ? panel : partials);
 }
 
 // m <= 64 takes the skinny kernel.  Larger m takes the kernel and tile with the

@@ -103,6 +103,9 @@ int fh_hip_fail(fh_ctx* ctx, hipError_t e, const char* what);
 
 // Make sure ctx->ws holds at least `bytes` (device, 256-B aligned).
 int fh_workspace(fh_ctx* ctx, size_t bytes, void** out);
+// Grow ctx->ws to `bytes` for later calls if that can be done now (not under graph
+// capture); this call does not depend on it.
+void fh_reserve_workspace(fh_ctx* ctx, size_t bytes);
 // The same for ctx->act.
 int fh_act_area(fh_ctx* ctx, size_t bytes, void** out);
 // Make sure ctx->sync holds at least `bytes`, zeroed when (re)allocated.
@@ -175,6 +178,14 @@ int fh_launch_skinny_scratch(fh_ctx* ctx, const fh_q8_0* w, const float* x, size
 // W8A8 (fast: FH_W8A8_FAST, each block term fused into the sum by one FMA).
 int fh_launch_gemm_w8a8(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m,
                         const float* bias, float* y, bool fast);
+// Estimated ns of the int8 matrix-core GEMM in 64 x 64 tiles, encode included.
+size_t fh_w8a8_tile_ns(size_t m, size_t n, size_t kb, bool fast);
+// The most workspace that a W8A8 linear of up to m rows over k inputs asks for: an
+// encoded panel of whole 64-row tiles, from 256 rows of whole 256-row ones.
+static inline size_t fh_w8a8_workspace(size_t m, size_t k) {
+    const size_t rows = m < 256 ? (m + 63) / 64 * 64 : (m + 255) / 256 * 256;
+    return fh_align256(rows * k) + fh_align256(rows * (k / 32) * 4);
+}
 int fh_launch_linear_w8a8(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m,
                           const float* bias, float* y, bool fast);
 // FH_W8A32_EXACT: ferrum_core's sequential sums, bit for bit (no K split).

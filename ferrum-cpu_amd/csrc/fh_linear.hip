@@ -38,12 +38,11 @@ namespace {
 
 constexpr int kWaves = 4;  // waves per block of the GEMV with the LayerNorm prologue (the plain GEMV: one)
 constexpr int kLnMaxK = 2048;  // widest row the GEMV's LayerNorm prologue takes
-// W8A8 runs on the int8 matrix cores (every Q8_0 block of an output in order)
-// from this many outputs, or this many tiles of (32 or 64) x 64; fewer waves,
-// each walking all of K, lose to the block-parallel kernel below (768 x 3072:
-// 19.3 against 26.4 us at m = 64, 32.6 against 26.8 at 128; 2304 x 768: 10.4
-// against 10.9 at 32, 15.4 against 11.7 at 64).
-constexpr size_t kW8a8MfmaOutputs = 96 * 1024, kW8a8MfmaTiles = 96;
+// W8A8 runs on the int8 matrix cores (every Q8_0 block of an output in order, the
+// reference's bits) from 32 rows and this many tiles of (32 or 64) x 64, and from 8
+// rows where they should take less time than the block-parallel kernel below
+// (fh_launch_linear_w8a8).
+constexpr size_t kW8a8MfmaTiles = 96;
 
 __device__ __forceinline__ float sbyte(uint32_t w, int i) {
     return static_cast<float>(static_cast<int8_t>((w >> (8 * i)) & 0xFFu));
@@ -460,10 +459,21 @@ int fh_launch_linear_w8a8(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t 
     if (w->n > 0x7FFFFFFFu || w->k > 0x7FFFFFFFu || m * w->n > 0x7FFFFFFFu * size_t(64))
         return fh_fail(ctx, FH_ERR_LIMIT, "fh_q8_0_linear: problem too large for the W8A8 kernel");
     const size_t tile_rows = m >= 64 ? 64 : 32;
-    if ((m >= 8 && m * w->n >= kW8a8MfmaOutputs) ||
-        (m >= 32 && (m + tile_rows - 1) / tile_rows * ((w->n + 63) / 64) >= kW8a8MfmaTiles))
-        return fh_launch_gemm_w8a8(ctx, w, x, m, bias, y, fast);
     const size_t kb = w->k / 32;
+    // The block-parallel kernel: its waves issue, per step, g lanes of every output.
+    // Fitted with fh_w8a8_tile_ns.  (6 %: what the matrix cores' in-order sums, the
+    // reference's bits, may cost.)  us, block-parallel and matrix cores: 768 x 3072 at
+    // m = 96 26.2 / 30.0, at 128 32.8 / 30.0; 3072 x 1024 at m = 32 12.5 / 14.7, at 48
+    // 15.7 / 14.6; 9728 x 896 at m = 8 11.0 / 12.3, at 16 16.1 / 12.8; 801 x 288 at m = 96
+    // 7.9 / 9.9, at 200 10.4 / 10.0.  (50257 x 768 at m = 6 38.9 / 17.4: fewer than 8 rows
+    // have always kept the parallel sums.)
+    const size_t g = kb >= 64 ? 64 : kb >= 16 ? 16 : kb >= 4 ? 4 : 1;
+    const double parallel_ns = 6100 + static_cast<double>(m) * static_cast<double>(w->n) *
+                                          static_cast<double>(g * (61 + 183 * ((kb + g - 1) / g))) / 100000;
+    if ((m >= 32 && (m + tile_rows - 1) / tile_rows * ((w->n + 63) / 64) >= kW8a8MfmaTiles) ||
+        (m >= 8 && static_cast<double>(fh_w8a8_tile_ns(m, w->n, kb, fast)) < 1.06 * parallel_ns))
+        return fh_launch_gemm_w8a8(ctx, w, x, m, bias, y, fast);
+    if (m >= 8) fh_reserve_workspace(ctx, fh_w8a8_workspace(m, w->k));
     const size_t qbytes = fh_align256(m * w->k), dbytes = fh_align256(m * kb * 2);
     void* ws = nullptr;
     int rc = fh_workspace(ctx, qbytes + dbytes, &ws);

@@ -101,3 +101,28 @@ def test_shorter_prompts_after_the_longest(orc, n, k, longest, m):
         out = torch.empty((m, n), device="cuda")
         replays_equal_eager(ctx, lambda: ferrum_hip.linear_forward_async(ctx, w, x, m, k, b, n, out), out)
         w.free()
+
+
+# W8A8: after a call of a few outputs at m rows (the block-parallel kernel), one of
+# many outputs (the matrix cores, whose panel has whole 64-row tiles) needs no more
+# workspace, nor does any of fewer rows.
+@pytest.mark.parametrize("numerics", ["W8A8", "W8A8_FAST"])
+@pytest.mark.parametrize("m1,m2", [(20, 20), (31, 9), (511, 300)])
+def test_w8a8_of_wider_outputs_after_narrow_ones(orc, numerics, m1, m2):
+    import torch
+
+    import ferrum_hip
+
+    k, mode, rng = 2048, getattr(ferrum_hip, numerics), np.random.default_rng(m1)
+    with fresh_context() as ctx:
+        wide = ferrum_hip.Q8_0Weight.upload(ctx, orc.quantize_weight(30000, k, 1, 0.05), 30000, k)
+        narrow = ferrum_hip.Q8_0Weight.upload(ctx, orc.quantize_weight(64, k, 2, 0.05), 64, k)
+        x, = on_device(rng.standard_normal((m1, k)).astype(np.float32))
+        y = torch.empty((m1, 64), device="cuda")
+        torch.cuda.synchronize()
+        ferrum_hip.linear_forward_async(ctx, narrow, x, m1, k, None, 0, y, mode)
+        ctx.sync()
+        out = torch.empty((m2, 30000), device="cuda")
+        replays_equal_eager(ctx, lambda: ferrum_hip.linear_forward_async(ctx, wide, x, m2, k, None, 0, out, mode), out)
+        wide.free()
+        narrow.free()

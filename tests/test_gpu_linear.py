@@ -527,10 +527,8 @@ def test_w8a8_matrix_cores_are_bit_exact(fh, orc, m, n, k, has_bias):
     matrix cores (one v_mfma_i32_32x32x32_i8 per Q8_0 block of a 32 x 32
     tile) and adds the scaled block dots in the reference's order without FMA:
     equal to the reference bit for bit, non-finite rows, ragged shapes and
-    odd block counts included.  From m = 1024 the operands go through LDS
-    (256 x 256 workgroup tiles) as f16, the block dot is two f16 MFMAs (an
-    exact integer in f32) and d_w * d_x one f32 outer-product MFMA: rows and
-    columns past a tile edge, one block and an odd number of blocks."""
+    odd block counts included.  All of these take the 64 x 64 workgroup tiles
+    (the 256 x 256 ones: test_w8a8_on_the_256_tiles)."""
     import ferrum_hip
 
     raw = weight(orc, n, k, 7 * m + n + k)
@@ -553,7 +551,7 @@ def test_w8a8_matrix_cores_are_bit_exact(fh, orc, m, n, k, has_bias):
 def test_w8a8_takes_rows_at_a_4_byte_offset(fh, orc, m, n, k):
     """x need only be 4-byte aligned: from a torch view one float into its
     buffer the panel encoder reads it with 4-byte loads, and the outputs still
-    equal the reference bit for bit (the matrix-core path and the staged one)."""
+    equal the reference bit for bit."""
     import torch
 
     import ferrum_hip
@@ -581,8 +579,8 @@ def test_w8a8_fast_is_within_the_rule_of_w8a8(fh, orc, m, n, k, has_bias):
     block's term fused into the sum (one FMA): within 1e-5 of the reference's
     W8A8 outputs relative to the magnitudes of the block terms summed, the same
     inf/NaN pattern, and at least as accurate as W8A8 against the float64 sum
-    of the same terms.  The matrix-core kernel (from 96 output tiles), the
-    staged one (m >= 1024) and the block-parallel kernel (below 96 tiles)."""
+    of the same terms.  The matrix-core kernel in 64 x 64 tiles (from 96
+    output tiles) and the block-parallel kernel (below 96 tiles)."""
     import ferrum_hip
 
     raw = weight(orc, n, k, 5 * m + n + k)
@@ -681,11 +679,11 @@ def test_q8_0_dequant_is_bit_exact(fh, orc):
     assert np.array_equal(out.cpu().numpy().view(np.uint32), orc.q8_0_dequant(raw, 32 * 5000).view(np.uint32))
 
 
-# The int8 matrix-core kernels' edges: one and odd block counts (K is walked in
-# pairs, four pairs in flight), ragged rows and columns, one and two 32-row
-# tiles per wave and the LDS-staged kernel, non-finite scales on either side:
-# the reference's bits.
-@pytest.mark.parametrize("m,n,k", [(8, 12321, 32), (33, 3010, 96), (127, 801, 288), (511, 1024, 160), (6081, 1, 64),
+# The int8 matrix-core kernel's edges: one and odd block counts (four blocks per
+# stage), ragged rows and columns, fewer than 32 rows of a wide output (and 8 x 12321
+# from one block, the block-parallel kernel, whose single term has the same bits),
+# non-finite scales on either side: the reference's bits.
+@pytest.mark.parametrize("m,n,k", [(8, 40001, 96), (9, 50257, 160), (31, 12288, 224), (8, 12321, 32), (33, 3010, 96), (127, 801, 288), (511, 1024, 160), (6081, 1, 64),
                                    (1000, 3073, 96), (2050, 2000, 224), (1025, 16129, 64)])
 def test_w8a8_pairs_of_blocks_are_bit_exact(fh, orc, m, n, k):
     import ferrum_hip
@@ -742,3 +740,52 @@ def test_prompt_rows_on_every_tile(fh, orc, m, n, k, gelu):
             want, mass = orc.gelu(want), 1.13 * mass  # |gelu'| <= 1.13 carries the linear's bound over
         assert np.array_equal(np.isnan(got[rows]), np.isnan(want))
         assert_close(np.where(finite, got[rows], 0), np.where(finite, want, 0), mass)
+
+
+def takes_the_256_tiles(m, n, k, fast, cus=256):
+    """fh_launch_gemm_w8a8's choice, from its two estimates in ns."""
+    kb, t32 = k // 32, -(-m // 32) * -(-n // 32)
+    chain = 5700 + 40 * min(m, 30) + (220 if fast else 240) * kb
+    chip = 4500 + t32 * (114 * kb + 750) // 1000 if fast else 6500 + t32 * (122 * kb + 730) // 1000
+    rounds = -(-(-(-m // 256) * -(-n // 256)) // cus)
+    return 7000 + rounds * (1520 * kb + 15300 if fast else 1880 * kb + 16300) < max(chain, chip)
+
+
+# The 256 x 256 tiles of W8A8 and of its fast mode, which take calls that nearly
+# fill whole rounds of the chip: one round of ragged rows and columns and an odd
+# number of blocks, and two rounds; non-finite scales on either side.  Sampled rows
+# against the oracle: bit for bit, and in the fast mode 1e-5 of the summed terms.
+@pytest.mark.parametrize("fast,m,n,k", [(False, 4090, 4081, 1632), (False, 8190, 4090, 1664), (True, 4090, 4081, 544),
+                                        (True, 3841, 4096, 1024)])
+def test_w8a8_on_the_256_tiles(fh, orc, fast, m, n, k):
+    import torch
+
+    import ferrum_hip
+
+    assert takes_the_256_tiles(m, n, k, fast) and not takes_the_256_tiles(1030, 700, 96, fast)
+    raw = orc.quantize_weight(n, k, m + n, 0.05)
+    raw.reshape(n, k // 32, 34)[n // 2, -1, :2] = np.array([np.inf], np.float16).view(np.uint8)
+    x = np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32)
+    x[m // 2, k - 1], x[m - 1, 0], x[300] = np.inf, np.nan, 0.0
+    b = np.random.default_rng(n).standard_normal(n).astype(np.float32)
+    w = ferrum_hip.Q8_0Weight.upload(fh, raw, n, k)
+    dx, db = torch.from_numpy(x).cuda(), torch.from_numpy(b).cuda()
+    y = torch.full((m, n), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    ferrum_hip.linear_forward_async(fh, w, dx, m, k, db, n, y,
+                                    ferrum_hip.W8A8_FAST if fast else ferrum_hip.W8A8)
+    fh.sync()
+    rows = [0, 31, 32, 127, 128, 255, 256, 300, m // 2, m - 250, m - 2, m - 1]
+    got = y.cpu().numpy()
+    w.free()
+    ref = orc.q8_0_linear_w8a8(x[rows], raw, n, b)
+    assert np.isfinite(got[300, :n // 2]).all()
+    if not fast:
+        assert np.array_equal(got[rows], ref, equal_nan=True)
+        return
+    assert np.array_equal(np.isnan(got[rows]), np.isnan(ref)) and np.array_equal(np.isinf(got[rows]), np.isinf(ref))
+    fin = np.isfinite(ref)
+    with np.errstate(invalid="ignore"):
+        mass = np.where(fin, term_mass(orc, x[rows], raw, n, k), 0)
+    # (a term's size from the activations as they are: the encoded ones are at most 1/254 larger)
+    assert_close(np.where(fin, got[rows], 0), np.where(fin, ref, 0), mass)
