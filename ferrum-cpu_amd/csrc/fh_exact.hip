@@ -47,7 +47,7 @@ struct Q8Src {
     __device__ __forceinline__ void store(int tid, int c, int k, const Raw& r, fh_seq::f4* wt) const {
         const int col = tid & 15, seg = tid >> 4;
         // past K: d = 0 (the products are +0 or -0, and a sum that starts at +0 is never -0)
-        const float d = c * kChunk + seg * 8 < k ? fh_h2f(r.d) : 0.0f;
+        const float d = fh_seq::inside(c, seg * 8, k) ? fh_h2f(r.d) : 0.0f;
         const uint32_t words[2] = {r.q.x, r.q.y};
 #pragma unroll
         for (int v = 0; v < 2; v++) {
@@ -98,7 +98,7 @@ struct F32Src {
     }
     __device__ __forceinline__ void store(int tid, int c, int k, const Raw& r, fh_seq::f4* wt) const {
         const int col = tid & 15, seg = tid >> 4;
-        const bool in = c * kChunk + seg * 8 < k;
+        const bool in = fh_seq::inside(c, seg * 8, k);
 #pragma unroll
         for (int v = 0; v < 2; v++)
             wt[(seg * 2 + v) * C + col] = in ? r.v[v] : fh_seq::f4{0.0f, 0.0f, 0.0f, 0.0f};

@@ -83,7 +83,7 @@ struct LevelSrc {
         const int g = tid >> 3, piece = tid & 7;
         uint32_t v[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = c * fh_seq::kChunk + 4 * g + i < k ? r.v[i] : 0u;
+        for (int i = 0; i < 4; i++) v[i] = fh_seq::inside(c, 4 * g + i, k) ? r.v[i] : 0u;
 #pragma unroll
         for (int h = 0; h < C / kBytes; h++)
 #pragma unroll
@@ -364,7 +364,7 @@ __global__ void __launch_bounds__(kThreads)
 // at m = 2 18.2 / 9.5, int4 50257 x 768 at m = 4 28.4 / 26.4 and at m = 5 32.0 / 44.3.
 bool few_rows(int kind, size_t cus, size_t pitch, size_t row_bytes, size_t k, size_t m, size_t cols) {
     const bool int8 = kind == FH_QINT8;
-    if (m > 64) return false;
+    if (m > 64 || k > 0x7FFFFC00u) return false;  // (k_qlinear's positions run up to a chunk past K in 32 bits)
     const double wgs = static_cast<double>(pitch / kTile * ((m + 3) / 4)) / static_cast<double>(cus);
     const double pairs = ceil(wgs / 2) - 1, rest = wgs - 2 * pairs;
     const bool crowded = int8 && pairs > 0 && k > kChunk;  // (chunks of several workgroups stream at once)

@@ -53,6 +53,16 @@ constexpr int kGroups = kChunk / 4;  // float4 groups per column and chunk
 constexpr int kPieces = kChunk / 16; // activation registers per row and chunk
 constexpr int kQueue = 4;            // products in flight per chain
 
+// Chunks of K.  (K goes up to 2^31 - 1: rounding it up first would overflow, and the
+// position after the last chunk is 2^31, so positions are compared unsigned.)
+__host__ __device__ constexpr int chunks_of(int k) { return (k - 1) / kChunk + 1; }
+static_assert(chunks_of(1) == 1 && chunks_of(kChunk) == 1 && chunks_of(kChunk + 1) == 2 &&
+                  chunks_of(0x7FFFFFFF) == (1 << 24) && chunks_of(0x7FFFFFE0) == (1 << 24),
+              "the last chunk of the longest K starts inside it");
+__device__ __forceinline__ bool inside(int chunk, int p, int k) {
+    return static_cast<unsigned>(chunk) * kChunk + static_cast<unsigned>(p) < static_cast<unsigned>(k);
+}
+
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 // Lane N's value of each 16-lane row.
@@ -102,7 +112,7 @@ __global__ void __launch_bounds__(kThreads)
     // where rows are [p][n], they read the same lines
     const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (tile >= tiles) return;
-    const int chunks = (k + kChunk - 1) / kChunk;
+    const int chunks = chunks_of(k);
     const int col = src.column(tile, lane % C, n);
     const float b0 = bias && col >= 0 ? bias[col] : 0.0f;
     for (long i0 = static_cast<long>(blockIdx.y) * kTileRows; i0 < m; i0 += static_cast<long>(gridDim.y) * kTileRows) {
@@ -120,7 +130,7 @@ __global__ void __launch_bounds__(kThreads)
         auto load_x = [&](auto S, int c) __attribute__((always_inline)) {
             if (!live) return;
             const int p0 = min(c, chunks - 1) * kChunk;
-            if (p0 + kChunk <= k) {
+            if (p0 <= k - kChunk) {
 #pragma unroll
                 for (int s = 0; s < kPieces; s++) {
                     if constexpr (Src::kScaled) sn[s] = src.scale(p0 + 16 * s + l16);
@@ -146,11 +156,11 @@ __global__ void __launch_bounds__(kThreads)
 #pragma unroll
                     for (int r = 0; r < TM; r++) a[S][s][r] = a[S][s][r] * sn[s];
             }
-            if (c * kChunk + kChunk > k) {
+            if (!inside(c, kChunk - 1, k)) {
 #pragma unroll
                 for (int s = 0; s < kPieces; s++)
 #pragma unroll
-                    for (int r = 0; r < TM; r++) a[S][s][r] = c * kChunk + 16 * s + l16 < k ? a[S][s][r] : -0.0f;
+                    for (int r = 0; r < TM; r++) a[S][s][r] = inside(c, 16 * s + l16, k) ? a[S][s][r] : -0.0f;
             }
         };
         auto sum = [&](auto S) __attribute__((always_inline)) {
