@@ -131,9 +131,8 @@ void launch(fh_ctx* ctx, const Src& src, const fh_q8_0* w, const float* x, size_
     // (the decode form's positions run up to a chunk past K in 32 bits)
     const bool decode = (m == 1 || (m <= 65535 && tiles * m <= per_cu * cus)) && w->k > kChunk && w->k <= 0x7FFFF000u;
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(m)),
-                           dim3(fh_seq::kThreads), 0, ctx->stream, src, x, bias, y, static_cast<int>(w->n),
-                           static_cast<int>(w->k));
+        hipLaunchKernelGGL(kernel, fh_seq::tile_grid(tiles, m), dim3(fh_seq::kThreads), 0, ctx->stream, src, x, bias, y,
+                           static_cast<int>(w->n), static_cast<int>(w->k));
     };
     if (!decode) fh_seq::launch(ctx, src, tiles, x, m, bias, y, w->n, w->k);
     else if (tiles > 2 * cus && w->k < 2048) go(fh_seq::k_linear_seq_row<Src, 1>);

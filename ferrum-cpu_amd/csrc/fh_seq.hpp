@@ -110,7 +110,7 @@ __global__ void __launch_bounds__(kThreads)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     // neighbouring tiles on one XCD (workgroups are dealt to the eight in turn):
     // where rows are [p][n], they read the same lines
-    const int tile = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    const int tile = blockIdx.z * gridDim.x + (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (tile >= tiles) return;
     const int chunks = chunks_of(k);
     const int col = src.column(tile, lane % C, n);
@@ -268,7 +268,8 @@ __global__ void __launch_bounds__(kThreads)
     constexpr int C = Src::C, kSegs = (kWaves - 1) * 4, kRowChunk = kSegs * 16 * JOBS, kRowGroups = kRowChunk / 4;
     static_assert(C == 16 && !Src::kBiasFirst && !Src::kScaled, "the plain sum of 16 columns");
     __shared__ f4 prod[2][kRowGroups * C];
-    const int tid = threadIdx.x, lane = tid & 63, c16 = tid & 15, tile = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, c16 = tid & 15, tile = blockIdx.z * gridDim.x + blockIdx.x;
+    if (tile > (n - 1) / C) return;
     const int chunks = (k + kRowChunk - 1) / kRowChunk;
     const float* xr = x + static_cast<size_t>(blockIdx.y) * k;
     // wave-uniform role (a scalar branch: every wave meets the same barriers)
@@ -359,6 +360,12 @@ __global__ void __launch_bounds__(kThreads)
 // waits: int4 4096 x 1024 at m = 127 runs 45.3 / 43.1 / 39.4 us with TM = 1 / 2 /
 // 4 (8, 4 and 2 whole rounds), 768 x 3072 41.8 / 41.7 / 67.7 (384, 192 and 96
 // workgroups).
+// Column tiles as grid.x and grid.z: a multiple of eight in x, and no more than HIP's
+// 2^32 threads in that dimension.
+inline dim3 tile_grid(size_t tiles, size_t y) {
+    const size_t most = size_t(1) << 23, x = tiles < most ? (tiles + 7) / 8 * 8 : most;
+    return dim3(static_cast<unsigned>(x), static_cast<unsigned>(y), static_cast<unsigned>((tiles + x - 1) / x));
+}
 inline size_t row_tiles(size_t cols, size_t m, size_t tm) { return (m + kThreads / cols * tm - 1) / (kThreads / cols * tm); }
 inline size_t rows_per_lane(size_t cus, size_t cols, size_t tiles, size_t m) {
     auto blocks = [&](size_t tm) { return tiles * row_tiles(cols, m, tm); };
@@ -375,8 +382,7 @@ void launch(fh_ctx* ctx, const Src& src, size_t tiles, const float* x, size_t m,
     const size_t tm = rows_per_lane(static_cast<size_t>(ctx->num_cus), Src::C, tiles, m);
     auto go = [&](auto kernel) {
         const size_t gy = row_tiles(Src::C, m, tm);
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((tiles + 7) / 8 * 8), static_cast<unsigned>(gy < 65535 ? gy : 65535)),
-                           dim3(kThreads), 0, ctx->stream, src, x, bias, y, static_cast<int>(m), static_cast<int>(n),
+        hipLaunchKernelGGL(kernel, tile_grid(tiles, gy < 65535 ? gy : 65535), dim3(kThreads), 0, ctx->stream, src, x, bias, y, static_cast<int>(m), static_cast<int>(n),
                            static_cast<int>(k), static_cast<int>(tiles));
     };
     if (tm == 4) go(k_linear_seq<Src, 4>);

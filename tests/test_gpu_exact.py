@@ -159,3 +159,34 @@ def test_exact_few_outputs(fh, orc, m, n, k, f32):
     got = ferrum_hip.linear_forward(fh, x, w, b, numerics=ferrum_hip.W8A32_EXACT)
     w.free()
     bits_equal(got, want)
+
+
+def test_exact_more_columns_than_one_grid_dimension_holds(fh, orc):
+    """2^28 and more outputs: their tiles of 16 columns, 256 threads each, pass
+    what one grid dimension can count.  The weight repeats 4093 rows, so the
+    outputs repeat the oracle's."""
+    import torch
+
+    import ferrum_hip
+
+    n, k, period = (1 << 28) + 23, 32, 4093
+    raw = orc.quantize_weight(period, k, 5, 0.05)
+    x = np.random.default_rng(28).standard_normal((1, k), dtype=np.float32)
+    want = torch.from_numpy(reference(orc, x, raw, period, k, None)).cuda().ravel()
+    rows = torch.from_numpy(np.ascontiguousarray(raw).view(np.uint8).reshape(period, 34)).cuda()
+    wide = rows.repeat(n // period + 1, 1)[:n].contiguous()
+    torch.cuda.synchronize()
+    w = ferrum_hip.Q8_0Weight.upload_device(fh, wide, n, k)
+    fh.sync()
+    del wide
+    y = torch.full((n,), float("nan"), device="cuda")
+    dx = torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    ferrum_hip.linear_forward_async(fh, w, dx, 1, k, None, 0, y, ferrum_hip.W8A32_EXACT)
+    fh.sync()
+    w.free()
+    whole = n // period * period
+    assert torch.equal(y[:whole].view(-1, period), want.expand(whole // period, period))
+    assert torch.equal(y[whole:], want[:n - whole])
+    del y
+    torch.cuda.empty_cache()
