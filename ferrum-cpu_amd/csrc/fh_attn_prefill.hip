@@ -9,7 +9,7 @@
 // before the block come from the caches, the block's own from its q|k|v rows;
 // the same launch writes the block's k / v rows into the caches.
 //
-// How (head width 64): one workgroup per (128 query rows, head, sequence).
+// How (head widths 32 and 64): one workgroup per (128 query rows, head, sequence).
 // Each of its four waves owns 32 query rows and walks 32-key tiles of the
 // sequence's cache up to its last row's position; the tiles are staged in LDS
 // once for the four waves (double-buffered, the next tile's loads in flight
@@ -18,8 +18,9 @@
 // (exact rescaling between tiles), then O += P V on the matrix cores, P
 // going in straight from the S^T accumulators as the B operand of O^T += V^T P^T,
 // so that a lane keeps to one query throughout: the rescaling and the final
-// division are by its own factors.  The f32 operands ride on the
-// f16 matrix cores as two terms each (k_attn_prefill_f16 below).
+// division are by its own factors.  At width 64 the f32 operands ride on the
+// f16 matrix cores as two terms each (k_attn_prefill_f16 below); at width 32 they stay
+// as they are, on the fp32 ones (k_attn_prefill_f32).
 #include "fh_internal.hpp"
 
 #pragma clang fp contract(off)
@@ -28,13 +29,13 @@ namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr int kHd = 64;        // head width
+constexpr int kHd = 64;        // k_attn_prefill_f16's head width
 constexpr int kKeys = 32;      // keys per tile
 constexpr int kRT = 4;         // waves of 32 query rows that share a key tile
 constexpr int kPT = 64 * kRT, kQRows = 32 * kRT;
 
 struct PrefillArgs {
-    const float* qkv;   // row s * rows + r; head h's q at column h * 64
+    const float* qkv;   // row s * rows + r; head h's q at column h * hd
     int ld;             // qkv row stride (floats)
     float* kc;          // sequence s's caches at kc / vc + s * seq_stride, rows of kv_dim floats
     float* vc;
@@ -42,7 +43,7 @@ struct PrefillArgs {
     int kv_dim;
     int rows, pos0;
     float scale;
-    float* out;         // row s * rows + r; head h at column h * 64
+    float* out;         // row s * rows + r; head h at column h * hd
     int out_ld;
 };
 
@@ -471,28 +472,245 @@ __global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f16(PrefillArgs
                 make_float4(o[d][4 * a4] / l, o[d][4 * a4 + 1] / l, o[d][4 * a4 + 2] / l, o[d][4 * a4 + 3] / l);
 }
 
+// e^x for x <= 0 as 2^(x log2 e), the product's rounding carried along: about 1 ulp.
+__device__ __forceinline__ float exp_f32(float x) {
+    x = x < -120.0f ? -120.0f : x;  // (NaN stays; 2^-173 is 0)
+    const float t = x * 1.44269504088896341f;
+    const float r = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269504088896341f, -t));
+    const float e = __builtin_amdgcn_exp2f(t);
+    return fmaf(e * r, 0.693147180559945f, e);
+}
+
+// Head width 32, on the fp32 matrix cores: the same walk, every operand as it is.
+// S^T = K Q^T and O^T += V^T P^T are 16 v_mfma_f32_32x32x2_f32 each per 32-key tile (a
+// step takes one dim of either half of the width, or one key of either half of the
+// wave, as A and B).  The v tile is staged as it lies.  Sums in short chains, a
+// tile's own products before the running sum: error against float64 over 17 shapes
+// 8.4e-8, 1.19e-7 at most (the vector-unit kernel 8.8e-8 and 1.24e-7; two f16 terms per
+// operand 1.27e-7 and 2.4e-7, and 3.2e-6 with v a hundredth as large, whose terms hold
+// 2^-25 and no less).
+// A tile with inf or NaN in v takes only the attended keys, on the vector units: 0 *
+// inf would turn a masked key's v into NaN.
+// Bound: the matrix cores, 32 products of 64 cycles per tile, and some 350 vector
+// instructions beside them.  us, d = 1024 and 32 heads: 16 prompts of 128 rows 19.3, 32
+// of 500 rows 251 (vector units, one sequence at a time: 350, 10069); d = 128 with 4
+// heads, 32 of 64 rows: 7.1 (182).
+template <int HALVES>
+__global__ void __launch_bounds__(kPT* HALVES, 2) k_attn_prefill_f32(PrefillArgs a) {
+    constexpr int W = 32, kKP = W + 4, kVP = W + 8;  // pitches: 16-byte pieces of 16 keys, and two keys 4 apart, on different banks
+    struct Stage {
+        __align__(16) float k[2][kKeys * kKP], v[2][kKeys * kVP];
+        int unsafe[3];  // a tile's v is not all finite (step st: st % 3)
+    };
+    __shared__ Stage stages[HALVES];
+    static_assert(HALVES == 1 || sizeof(Stage) >= kRT * 18 * 64 * sizeof(float), "the merge fits a stage");
+    const int hf = HALVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kPT);
+    Stage& sm = stages[hf];
+    const int tid = threadIdx.x % kPT, lane = tid & 63, half = lane >> 5, col = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int groups = static_cast<int>(gridDim.z), g = groups - 1 - static_cast<int>(blockIdx.z);
+    const int h = blockIdx.x, s = blockIdx.y;
+    const int r0 = g * kQRows + wave * 32;
+    const int kmax = a.pos0 + min(a.rows - 1, g * kQRows + kQRows - 1);
+    const int ntiles = kmax / kKeys + 1;
+    const int my_tiles = r0 < a.rows ? (a.pos0 + min(a.rows - 1, r0 + 31)) / kKeys + 1 : 0;
+    const size_t sbase = static_cast<size_t>(s) * a.seq_stride + static_cast<size_t>(h) * W;
+    float* kc = a.kc + sbase;
+    float* vc = a.vc + sbase;
+    const float* bq = a.qkv + static_cast<size_t>(s) * a.rows * a.ld + h * W;  // this sequence's block rows
+
+    // this lane's query, dims 16 half + (0..15): step i of a score is dims i and 16 + i
+    float q[16];
+    {
+        const float* qp = bq + static_cast<size_t>(min(r0 + col, a.rows - 1)) * a.ld + half * 16;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float4 u = *reinterpret_cast<const float4*>(qp + 4 * i);
+            q[4 * i] = u.x; q[4 * i + 1] = u.y; q[4 * i + 2] = u.z; q[4 * i + 3] = u.w;
+        }
+    }
+    const int qpos = a.pos0 + r0 + col;
+
+    // Staging: thread t takes 16 bytes of k and of v of key t / 8.  The last row group's
+    // workgroup of each (sequence, head) also writes the block's rows into the caches.
+    const bool writer = g == groups - 1;
+    const int key_of = tid / 8, c0 = tid % 8 * 4;
+    float4 pk, pv;
+    auto fetch = [&](int t) __attribute__((always_inline)) {
+        const int key = min(t * kKeys + key_of, kmax);
+        const bool own = key >= a.pos0;
+        const float* row = bq + static_cast<size_t>(max(key - a.pos0, 0)) * a.ld + c0;
+        const size_t at = static_cast<size_t>(key) * a.kv_dim + c0;
+        pk = *reinterpret_cast<const float4*>(own ? row + a.kv_dim : kc + at);
+        pv = *reinterpret_cast<const float4*>(own ? row + 2 * a.kv_dim : vc + at);
+    };
+    auto store_block_rows = [&](int t) __attribute__((always_inline)) {
+        const int key = t * kKeys + key_of;
+        if (key < a.pos0 || key > kmax) return;
+        const size_t at = static_cast<size_t>(key) * a.kv_dim + c0;
+        *reinterpret_cast<float4*>(kc + at) = pk;
+        *reinterpret_cast<float4*>(vc + at) = pv;
+    };
+    auto stash = [&](int st) __attribute__((always_inline)) {
+        *reinterpret_cast<float4*>(&sm.k[st & 1][key_of * kKP + c0]) = pk;
+        *reinterpret_cast<float4*>(&sm.v[st & 1][key_of * kVP + c0]) = pv;
+        const bool finite = __builtin_isfinite(pv.x) && __builtin_isfinite(pv.y) && __builtin_isfinite(pv.z) &&
+                            __builtin_isfinite(pv.w);
+        if (__builtin_expect(!finite, 0)) sm.unsafe[st % 3] = 1;
+    };
+
+    float m_run = -INFINITY, l_run = 0.0f;
+    f32x16 o = f32x16{};
+    const int steps = (ntiles + HALVES - 1) / HALVES;
+    if (tid < 3) sm.unsafe[tid] = 0;
+    fetch(hf);
+    if (writer) store_block_rows(hf);
+    __syncthreads();
+    stash(0);
+    __syncthreads();
+    for (int st = 0; st < steps; st++) {
+        const int t = st * HALVES + hf, tn = t + HALVES, k0 = t * kKeys;
+        if (tn < ntiles) fetch(tn);
+        const bool vbad = sm.unsafe[st % 3] != 0;
+        if (tid == 0) sm.unsafe[(st + 2) % 3] = 0;  // (read at step st - 1, written next at step st + 1)
+        if (t < my_tiles) {
+            const float* kt = sm.k[st & 1] + col * kKP + half * 16;
+            const float* vt = sm.v[st & 1];
+            f32x16 sacc[2] = {f32x16{}, f32x16{}};  // (two chains: fewer roundings in a row)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float4 u = *reinterpret_cast<const float4*>(kt + 4 * i);
+                sacc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(u.x, q[4 * i], sacc[0], 0, 0, 0);
+                sacc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(u.y, q[4 * i + 1], sacc[1], 0, 0, 0);
+                sacc[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(u.z, q[4 * i + 2], sacc[0], 0, 0, 0);
+                sacc[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(u.w, q[4 * i + 3], sacc[1], 0, 0, 0);
+            }
+            float sv[16], mt = -INFINITY;
+#pragma unroll
+            for (int v = 0; v < 16; v++) sv[v] = (sacc[0][v] + sacc[1][v]) * a.scale;
+            if (k0 + kKeys - 1 > a.pos0 + r0)
+#pragma unroll
+                for (int v = 0; v < 16; v++) sv[v] = k0 + acc_row(v, half) <= qpos ? sv[v] : -INFINITY;
+#pragma unroll
+            for (int v = 0; v < 16; v++) mt = fmaxf(mt, sv[v]);
+            // (a query whose scores so far are all -inf keeps sums of 0, and 0 / 0 = NaN)
+            const float m_new = fmaxf(m_run, max_halves(mt)), m_exp = m_new == -INFINITY ? 0.0f : m_new;
+            const float corr = exp_f32(m_run - m_exp);  // 0 on the first tile (m_run = -inf)
+            float ps[4] = {};
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                sv[v] = exp_f32(sv[v] - m_exp);
+                ps[v & 3] += sv[v];
+            }
+            // (this half's keys; the halves are added at the end)
+            l_run = fmaf(l_run, corr, (ps[0] + ps[1]) + (ps[2] + ps[3]));
+            m_run = m_new;
+            if (!vbad) {
+                // (the tile's own sum first: a running sum of all keys' products would
+                // round once per key instead of once per tile)
+                f32x16 first;
+#pragma unroll
+                for (int v0 = 0; v0 < 16; v0 += 8) {
+                    f32x16 ot[2] = {f32x16{}, f32x16{}};
+#pragma unroll
+                    for (int v = v0; v < v0 + 8; v++)
+                        ot[v & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vt[acc_row(v, half) * kVP + col], sv[v], ot[v & 1], 0, 0, 0);
+                    if (v0 == 0) first = ot[0] + ot[1];
+                    else
+#pragma unroll
+                        for (int d = 0; d < 16; d++) o[d] = fmaf(o[d], corr, first[d] + (ot[0][d] + ot[1][d]));
+                }
+            } else {
+                o *= corr;
+                // (keys past the query's position, or past the block's last one, are left out)
+                const int last = min(qpos, kmax);
+#pragma unroll
+                for (int v = 0; v < 16; v++) {
+                    const float other = __shfl_xor(sv[v], 32, 64);
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        const int key = acc_row(v, e);
+                        const float p = e == half ? sv[v] : other;
+                        if (k0 + key <= last)
+#pragma unroll
+                            for (int d = 0; d < 16; d++) o[d] += p * vt[key * kVP + acc_row(d, half)];
+                    }
+                }
+            }
+        }
+        if (tn < ntiles) {
+            if (writer) store_block_rows(tn);
+            stash(st + 1);
+        }
+        __syncthreads();
+    }
+    float l = l_run + __shfl_xor(l_run, 32, 64);
+    if constexpr (HALVES == 2) {
+        // the odd tiles' maximum, sum and outputs, scaled to the common maximum
+        float* mg = reinterpret_cast<float*>(&stages[1]) + wave * (18 * 64) + lane;
+        if (hf == 1) {
+            mg[0] = m_run;
+            mg[64] = l;
+#pragma unroll
+            for (int v = 0; v < 16; v++) mg[(2 + v) * 64] = o[v];
+        }
+        __syncthreads();
+        if (hf == 1) return;
+        const float m1 = mg[0], m = fmaxf(m_run, m1), m_exp = m == -INFINITY ? 0.0f : m;
+        const float f0 = exp_f32(m_run - m_exp), f1 = exp_f32(m1 - m_exp);
+        l = l * f0 + mg[64] * f1;
+#pragma unroll
+        for (int v = 0; v < 16; v++) o[v] = o[v] * f0 + mg[(2 + v) * 64] * f1;
+    }
+    const int row = r0 + col;
+    if (row >= a.rows) return;
+    float* op = a.out + (static_cast<size_t>(s) * a.rows + row) * a.out_ld + h * W + half * 4;
+#pragma unroll
+    for (int a4 = 0; a4 < 4; a4++)
+        *reinterpret_cast<float4*>(op + 8 * a4) =
+            make_float4(o[4 * a4] / l, o[4 * a4 + 1] / l, o[4 * a4 + 2] / l, o[4 * a4 + 3] / l);
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// Head width 32: whether the vector-unit kernel, two launches per sequence, should take
+// less than the matrix cores' `ns`, as it does for one or a few sequences with many
+// earlier positions, whose key tiles are one workgroup's chain: one row after 700, 4
+// heads 7.9 us against 38, 128 rows 18.2 / 47; four of them 70.5 / 48.  A sequence takes
+// 6.2 us, or 5.7 and 2.7 ns per workgroup with keys to attend (one for each row, head
+// and 64 positions, 128 from 769 on), or so much per workgroup launched where the
+// chunks of a row are a multiple of 4 or 8, which deals the later, often empty ones to
+// the same XCDs.  It keeps partial sums in the context's areas, so a call under graph
+// capture that they do not hold stays on the matrix cores.
+bool few_sequences(fh_ctx* ctx, size_t heads, size_t pos0, size_t rows, size_t seqs, size_t ns) {
+    const size_t len = pos0 + rows, keys = len > 768 ? 128 : len > 32 ? 64 : 32, chunks = (len + keys - 1) / keys;
+    const size_t busy = heads * rows * (2 * pos0 + rows + keys) / (2 * keys) * (chunks == 1 ? 100 : 270) / 100;
+    const size_t all = heads * rows * chunks * (chunks % 8 == 0 ? 300 : chunks % 4 == 0 ? 215 : 0) / 100;
+    const size_t work = 5700 + (busy > all ? busy : all);
+    if (1500 + seqs * (work > 6200 ? work : 6200) >= ns) return false;
+    if (ctx->ws_bytes >= heads * rows * chunks * 34 * sizeof(float) && ctx->counters_bytes >= heads * rows * sizeof(unsigned))
+        return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+}
 
 }  // namespace
 
 int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, float* vc, size_t seq_stride,
                                      size_t d, size_t heads, size_t pos0, size_t rows, size_t seqs, float* out) {
     const size_t hd = d / heads;
-    const bool mfma = hd == static_cast<size_t>(kHd) && aligned16(qkv) && aligned16(kc) && aligned16(vc) &&
+    const bool mfma = (hd == 32 || hd == static_cast<size_t>(kHd)) && aligned16(qkv) && aligned16(kc) && aligned16(vc) &&
                       aligned16(out) && seq_stride % 4 == 0;
-    if (!mfma) {
-        // other head widths: the vector-unit kernel, one sequence at a time.
-        // (Not width 32 either: there the two f16 terms lose bits that it keeps,
-        // 1.27e-7 of float64 against 8.8e-8 over 17 shapes, and 3.2e-6 against 8.8e-8
-        // with v a hundredth as large; and a row after 700 cached ones took 23.9 us
-        // against 8.0, its chain of tiles being one workgroup's.)
+    // (one sequence at a time)
+    auto on_vector_units = [&]() -> int {
         for (size_t s = 0; s < seqs; s++) {
             const int rc = fh_launch_attention_prefill(ctx, qkv + s * rows * 3 * d, kc + s * seq_stride,
                                                        vc + s * seq_stride, d, heads, pos0, rows, out + s * rows * d);
             if (rc) return rc;
         }
         return FH_OK;
-    }
+    };
+    if (!mfma) return on_vector_units();  // other head widths
     PrefillArgs a{};
     a.qkv = qkv;
     a.ld = static_cast<int>(3 * d);
@@ -506,23 +724,29 @@ int fh_launch_attention_prefill_seqs(fh_ctx* ctx, const float* qkv, float* kc, f
     a.out = out;
     a.out_ld = static_cast<int>(d);
     const size_t cus = static_cast<size_t>(ctx->num_cus), pairs = heads * seqs, groups = (rows + kQRows - 1) / kQRows;
-    // One or two chains of key tiles per row.  Measured (ns): a
+    // One or two chains of key tiles per row.  Measured (ns) at head width 64: a
     // workgroup takes 2200 per tile alone on its CU, a CU of two 1750 per tile;
     // with two chains 1500 alone (one workgroup per CU) and 2300, and 1500 for the
     // merge.  8 sequences of 300 rows and 12 heads (288 workgroups of 4, 8 and 10
     // tiles): 25.2 us and 22.5; 16 heads: 25.7 and 27.5; one of 511 rows: 33.4 and
-    // 25.6; 32 of 511: 106.8 and 131.4.
+    // 25.6; 32 of 511: 106.8 and 131.4.  At width 32 1950 and 1550, 1600 and 1950: one
+    // sequence of 900 rows 60.0 us and 52.7, 32 of 500 rows and 32 heads 251 and 317.
+    const size_t tile1 = hd == 32 ? 1950 : 2200, tile2 = hd == 32 ? 1550 : 1750;
+    const size_t half1 = hd == 32 ? 1600 : 1500, half2 = hd == 32 ? 1950 : 2300;
     size_t tiles = 0;
     for (size_t g = 1; g <= groups; g++) tiles += (pos0 + (g * kQRows < rows ? g * kQRows : rows) - 1) / kKeys + 1;
     const size_t longest = (pos0 + rows - 1) / kKeys + 1, share = tiles * pairs / cus;
-    const size_t one = longest * 2200 > share * 1750 ? longest * 2200 : share * 1750;
-    const size_t two = (longest * 1500 > share * 2300 ? longest * 1500 : share * 2300) + 1500;
+    const size_t one = longest * tile1 > share * tile2 ? longest * tile1 : share * tile2;
+    const size_t two = (longest * half1 > share * half2 ? longest * half1 : share * half2) + 1500;
+    if (hd == 32 && few_sequences(ctx, heads, pos0, rows, seqs, 3300 + (one < two ? one : two)))
+        return on_vector_units();
     auto go = [&](auto kern, int halves) {
         // (at most 65535 sequences and 512 groups of rows: the callers' limits)
         hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(heads), static_cast<unsigned>(seqs), static_cast<unsigned>(groups)),
                            dim3(static_cast<unsigned>(kPT * halves)), 0, ctx->stream, a);
     };
-    two < one ? go(k_attn_prefill_f16<2>, 2) : go(k_attn_prefill_f16<1>, 1);
+    if (hd == 32) two < one ? go(k_attn_prefill_f32<2>, 2) : go(k_attn_prefill_f32<1>, 1);
+    else two < one ? go(k_attn_prefill_f16<2>, 2) : go(k_attn_prefill_f16<1>, 1);
     FH_HIP(ctx, hipGetLastError());
     return FH_OK;
 }

@@ -791,8 +791,8 @@ def test_config1_greedy_run_on_the_device(fh, orc):
 
 
 # The prompt attention's one and two chains of key tiles (by the launch's size)
-# at head width 64, and the vector-unit kernel at width 32: rows and earlier
-# positions on and beside the 32-key and 128-row tiles (a row whose keys all lie in the even tiles, tiles that a query
+# at head widths 64 and 32 (where one sequence of 130 rows goes to the vector units):
+# rows and earlier positions on and beside the 32-key and 128-row tiles (a row whose keys all lie in the even tiles, tiles that a query
 # does not reach), scores of -inf, and a tile whose v goes on the vector units.
 @pytest.mark.parametrize("d,heads", [(128, 2), (64, 2), (96, 3)])
 @pytest.mark.parametrize("seqs,rows,pos0", [(1, 1, 0), (1, 33, 31), (2, 65, 40), (1, 130, 0), (3, 129, 95), (260, 40, 1)])
@@ -854,13 +854,15 @@ def test_prompt_attention_large_v_in_the_last_ragged_tile(fh, orc, d, heads, row
             close(got[s * rows + r][fin], want[fin], 1e-5)
 
 
-# Head width 32 keeps f32's relative precision whatever the size of v: 1e-6 of the
+# Head width 32 keeps f32's relative precision whatever the size of v, on the fp32
+# matrix cores (two sequences and more) and on the vector units (one): 1e-6 of the
 # largest output (weights and sums of f32 give 1.3e-7; two f16 terms of v, which
 # hold 2^-25 and no less, 3e-4).
-def test_prompt_attention_of_small_v_at_width_32(fh):
+@pytest.mark.parametrize("seqs,rows", [(2, 130), (1, 130), (3, 700)])
+def test_prompt_attention_of_small_v_at_width_32(fh, seqs, rows):
     import ferrum_hip
 
-    d, heads, seqs, rows = 128, 4, 2, 130
+    d, heads = 128, 4
     rng = np.random.default_rng(32)
     qkv = (rng.standard_normal((seqs * rows, 3 * d)) * 0.55).astype(np.float32)
     qkv[:, 2 * d:] *= np.float32(1e-4)

@@ -126,3 +126,41 @@ def test_w8a8_of_wider_outputs_after_narrow_ones(orc, numerics, m1, m2):
         replays_equal_eager(ctx, lambda: ferrum_hip.linear_forward_async(ctx, wide, x, m2, k, None, 0, out, mode), out)
         wide.free()
         narrow.free()
+
+
+def test_prompt_attention_of_one_row_at_width_32(orc):
+    """Head width 32, one row after 700 positions: the vector units, whose partial
+    sums need the context's areas. Captured on a context that has none, it runs
+    on the matrix cores; either way within 1e-5 of the oracle."""
+    import torch
+
+    import ferrum_hip
+
+    d, heads, pos0 = 128, 4, 700
+    rng = np.random.default_rng(700)
+    qkv = rng.standard_normal((1, 3 * d)).astype(np.float32)
+    kc, vc = (rng.standard_normal((pos0 + 1, d)).astype(np.float32) for _ in range(2))
+    want = orc.attention_decode(qkv[0], kc.copy(), vc.copy(), heads, pos0)
+    with fresh_context() as ctx:
+        tq, tk, tv = on_device(qkv, kc, vc)
+        out = torch.empty((1, d), device="cuda")
+
+        def call():
+            ferrum_hip.attention_prefill_seqs_async(ctx, tq, tk, tv, 0, pos0 + 1, d, heads, pos0, 1, 1, out)
+
+        g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        try:
+            with torch.cuda.graph(g, stream=s):
+                ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+                call()
+        finally:
+            ctx.set_stream(None)
+        for run in (g.replay, call, g.replay, call, g.replay):
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            run()
+            ctx.sync()
+            torch.cuda.synchronize()
+            got = out.cpu().numpy()[0]
+            assert np.all(np.abs(got - want) <= 1e-5 * np.maximum(1.0, np.abs(want)))
