@@ -107,14 +107,19 @@ def test_exact_and_fast_modes_agree_to_the_rounding_rule(fh, orc):
     assert (np.abs(fast.astype(np.float64) - exact) <= 1e-5 * np.maximum(np.abs(exact), mass)).all()
 
 
-# One, two and four rows per lane (the launch rule takes more of them as the
-# tiles of 16 columns and 16 rows outnumber the CUs), each with a K that ends
+# One row per lane (tm = 1), and two and four, which the launch rule takes as the
+# tiles of 16 columns and 16 rows outnumber the CUs, each with a K that ends
 # inside a 128-position chunk or a 16-position piece of it, ragged rows and
 # columns.
-@pytest.mark.parametrize("m,n,k", [(16, 17, 128), (17, 16, 160), (33, 130, 352), (65, 4081, 96), (130, 4090, 160)])
+@pytest.mark.parametrize("m,n,k,tm", [(16, 17, 128, 1), (17, 16, 160, 1), (33, 130, 352, 1), (65, 4081, 96, 1),
+                                      (130, 4090, 160, 1), (63, 4090, 160, 2), (96, 4081, 352, 2), (125, 4090, 96, 4),
+                                      (128, 4081, 288, 4)])
 @pytest.mark.parametrize("f32", [False, True])
-def test_exact_rows_per_lane_and_ragged_edges(fh, orc, m, n, k, f32):
+def test_exact_rows_per_lane_and_ragged_edges(fh, orc, m, n, k, tm, f32):
     import ferrum_hip
+    import seq_tiles
+
+    assert seq_tiles.rows_per_lane(16, -(-n // 16), m) == tm
 
     rng = np.random.default_rng(m + n + k)
     k -= 7 if f32 else 0

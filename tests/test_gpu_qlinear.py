@@ -71,9 +71,9 @@ def test_qlinear_errors(fh, orc):
     w.free()
 
 
-# One, two and four rows per lane and both tile widths of the kernel for
-# several rows, K ending inside a chunk and inside a 16-position piece, odd
-# widths (the int4 halves' last columns), a bias of -0 under products of -0 (no
+# Both tile widths of the kernel for several rows (or k_qlinear, where the launch rule
+# takes it), one row per lane, K ending inside a chunk and inside a 16-position piece,
+# odd widths (the int4 halves' last columns), a bias of -0 under products of -0 (no
 # padding may turn the sum to +0) and non-finite activations.
 @pytest.mark.parametrize("kind", [0, 1])
 @pytest.mark.parametrize("m,k,n", [(2, 15, 1), (16, 128, 33), (17, 129, 31), (40, 300, 2303), (66, 130, 4095),
@@ -112,4 +112,18 @@ def test_qlinear_rows_per_lane_and_ragged_edges(fh, orc, kind, m, k, n):
                                         (0, 8, 513, 14337), (1, 2, 129, 32001), (1, 3, 100, 28673), (1, 4, 250, 28671),
                                         (1, 7, 129, 32001), (1, 8, 1025, 32767), (0, 4, 1537, 16384)])
 def test_qlinear_few_rows_of_a_wide_output(fh, orc, kind, m, k, n):
+    test_qlinear_rows_per_lane_and_ragged_edges(fh, orc, kind, m, k, n)
+
+
+# Two and four rows per lane, in tiles of 16 columns and of 32 (more than 64 rows never
+# take k_qlinear).
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("m,k,n,tm", [(95, 300, 4090, 2), (90, 129, 4089, 2), (125, 130, 4090, 4), (128, 97, 4095, 4),
+                                      (80, 70, 32769, 2), (78, 145, 32768, 2), (128, 33, 32769, 4), (123, 130, 32771, 4)])
+def test_qlinear_two_and_four_rows_per_lane(fh, orc, kind, m, k, n, tm):
+    import seq_tiles
+
+    cols, row_bytes = 32 if n >= 32768 else 16, n if kind == 0 else (n + 1) // 2
+    tiles = -(-row_bytes // (cols if kind == 0 else cols // 2))
+    assert seq_tiles.rows_per_lane(cols, tiles, m) == tm
     test_qlinear_rows_per_lane_and_ragged_edges(fh, orc, kind, m, k, n)
