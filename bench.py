@@ -874,7 +874,7 @@ def prefill_leg(ctx, fh, torch, gen, dev, steps):
                                "numerics": "W8A8 (activations re-quantised to Q8_0), bit-exact with the reference",
                                "roofline": {"bound": "mfma", "achieved": round(tops8, 1), "peak": I8_DENSE_TOPS,
                                             "unit": "TOP/s", "frac": round(tops8 / I8_DENSE_TOPS, 4), "traffic": None,
-                                            "kernel": "k_gemm_w8a8_lds (+ fh_k_encode_panel): 2 m n k ops of "
+                                            "kernel": "k_gemm_w8a8, k_gemm_w8a8_lds (+ fh_k_encode_panel): 2 m n k ops of "
                                                       "the int8 product per step of the 96 linears",
                                             "note": "bound by the reference's per-block rounding (a product and "
                                                     "a sum per output and block on the VALU): MFMA busy 29 %"}},

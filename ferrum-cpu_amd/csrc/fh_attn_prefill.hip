@@ -72,7 +72,7 @@ __device__ __forceinline__ int acc_row(int v, int half) { return (v >> 2) * 8 + 
 //     otherwise turn a masked key's v into NaN), v read from the cache.
 // The error is that of the 22-bit operands, ~2^-22 relative per product,
 // well inside the 1e-5 rule.
-// Bound: a wave's chain per tile, some 400 vector instructions, 24 dependent
+// Bound: a wave's chain per tile, some 550 vector instructions, 24 dependent
 // MFMAs and the waits for LDS and the barrier (a tile of its own keys: 790 vector
 // instructions, shuffles through LDS for every row maximum and an LDS round trip
 // for the rescaling before).  32 prompts of 511 rows, 12 heads: 176 -> 106 us, of
@@ -491,8 +491,8 @@ __device__ __forceinline__ float exp_f32(float x) {
 // 2^-25 and no less).
 // A tile with inf or NaN in v takes only the attended keys, on the vector units: 0 *
 // inf would turn a masked key's v into NaN.
-// Bound: the matrix cores, 32 products of 64 cycles per tile, and some 350 vector
-// instructions beside them.  us, d = 1024 and 32 heads: 16 prompts of 128 rows 19.3, 32
+// Bound: the matrix cores, 32 products of 64 cycles per tile (busy 47 % of the time over
+// 32 prompts of 500 rows), and some 410 vector instructions beside them.  us, d = 1024 and 32 heads: 16 prompts of 128 rows 19.3, 32
 // of 500 rows 251 (vector units, one sequence at a time: 350, 10069); d = 128 with 4
 // heads, 32 of 64 rows: 7.1 (182).
 template <int HALVES>

@@ -1535,8 +1535,9 @@ int launch_gemm(fh_ctx* ctx, const fh_q8_0* w, const float* x, size_t m, const f
 }
 
 // Splits of K only while the column tiles alone leave half the CUs idle, and
-// then as few as let one batch of BPW blocks per wave cover a split (each split
-// costs a round of partial stores and reloads).  Waves: at most 16 / (MT * NT)
+// then as few as let one batch of blocks per wave cover a split (each split costs a
+// round of partial stores and reloads): a batch of three where two or three are taken
+// at once, or one with two column tiles, else of one.  Waves: at most 16 / (MT * NT)
 // (their sums fit 64 KiB of LDS, two workgroups per CU) and 8 (256 VGPRs per lane).  Column tiles per
 // wave (NT): up to 4 while that still leaves >= 256 workgroups, so wide
 // outputs split each activation block once per 128 columns.
@@ -1814,8 +1815,8 @@ static void reserve_shorter_prompts(fh_ctx* ctx, size_t m, size_t k) {
 // least estimated time.  Fitted to timings over the GPT-2 and Qwen2-0.5B shapes
 // at m = 65 .. 16352 (256 CUs), with kb blocks of K:
 //  - the skinny kernel in row tiles of 32 (one 32 x 32 tile per workgroup, its
-//    waves splitting K: every load of a tile out at once): 4 us + kb * 0.42 ns per
-//    tile with four waves; with eight waves while two workgroups per CU hold all
+//    waves splitting K, one block each at a time): 4 us + kb * 0.42 ns per tile
+//    with four waves; with eight waves while two workgroups per CU hold all
 //    tiles;
 //  - the same in tiles of 64 x 64 (an activation block is split for 64 columns):
 //    5 us + kb * 620 ns per round of two workgroups per CU;

@@ -24,9 +24,10 @@
 
 namespace {
 
-// 12 MiB: the largest split-K layout the skinny GEMM picks for m <= 64 on a
-// 256-CU part is 127 tiles x 8 splits x 2048 outputs x 4 bytes (8.3 MB) plus
-// the counters; a shape that would need more is refused (FH_ERR_LIMIT).
+// 12 MiB: the plain skinny GEMM splits K while its 32 x 32 tiles, one or two row tiles
+// of them, number fewer than half the CUs: on a 256-CU part at most 127 tiles x 8
+// splits x 1024 outputs x 4 bytes (4.2 MB) plus the counters.  A shape that would
+// need more is refused (FH_ERR_LIMIT).
 constexpr size_t kFhNoallocScratchBytes = size_t(12) << 20;
 constexpr int kMaxDevices = 64;
 
